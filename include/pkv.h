@@ -49,9 +49,9 @@ typedef enum pkv_dtype {
                                 lighter workgroup so more of them are in flight at once */
 
 #define PKV_ATTN_DOMINANT_TILES 4 /* the tile pass carries more of the call's time than the row
-                                    pass beside it: run it as three register-staged workgroups
-                                    per CU (the row workgroups fill in around them) instead of
-                                    one (float32, staged straight into LDS) or two per CU */
+                                    pass beside it: run it as up to three workgroups per CU (the
+                                    row workgroups fill in around them) instead of one
+                                    (float32) or two */
 
 /* pkv_paged_attention tile record: end partition of a tile computed whole by one workgroup. */
 #define PKV_TILE_WHOLE (-1)
@@ -206,7 +206,7 @@ int pkv_tile_head_dim_supported(int32_t head_dim);
  *                      partitions up to an upper bound of the row's visible length is safe.
  *   tiles, num_tiles : the plan's tile list, int32 [num_tiles, 4] = (first row, row count <= 64,
  *                      first partition, end partition; end <= first means through the last):
- *                      runs of consecutive rows computed by the fp32 MFMA tile pass over those
+ *                      runs of consecutive rows computed by the MFMA tile pass over those
  *                      partitions, one workgroup per (tile, head, partition). Keys are read
  *                      through the table of the tile's first row, so the rows are either one
  *                      sequence's (a prefill chunk) or rows of several sequences whose tables

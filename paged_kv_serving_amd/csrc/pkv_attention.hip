@@ -14,13 +14,13 @@
 //     decode rows of several sequences over the partitions of a prefix they share): one
 //     workgroup per (tile of <= 64 rows, head, context partition). Keys are read through the
 //     table of the tile's first row, which the planner only allows where every row of the tile
-//     has the same blocks. Key and value tiles of 32 rows
-//     (16 at head_dim 256) are staged in LDS and shared by 4 wavefronts of 16 queries each:
-//     through registers into padded rows, or, for float32 pools beside the row pass, straight
-//     from HBM into three swizzled LDS stages (global_load_lds_dwordx4, two tiles in flight);
-//     the scores are computed as S^T = K Q^T and the output as O = P V with
-//     v_mfma_f32_16x16x4f32, so every lane owns four scores of one query per 16 keys and the P
-//     operand of the second product is the lane's own registers.
+//     has the same blocks. Key and value tiles of 32 rows are staged in LDS and shared by 4
+//     wavefronts of 16 queries each; the scores are computed as S^T = K Q^T and the output as
+//     O^T = V^T P^T, so every lane owns eight scores of one query per 32 keys and the P operand
+//     of the second product is the lane's own registers. The products run on
+//     v_mfma_f32_16x16x32_bf16 over exact bfloat16 pieces of the float32 operands; float32
+//     products (v_mfma_f32_16x16x4f32) remain for tiles that meet an infinity or NaN and for
+//     float32 tiles beside the lean row pass.
 //  3. reduce: rows whose visible context spans several partitions merge the per-partition
 //     (max, sum, acc) and write the normalised output. Rows that fit one partition were written
 //     by pass 1 or 2 directly.
@@ -44,10 +44,10 @@
 // and kept per device; host code never passes the array's own name to a kernel).
 static __device__ __align__(256) float scratch[PKV_STATIC_SCRATCH_BYTES / sizeof(float)];
 
-// Sixteen zero bytes in global memory: the tile pass loads the key and value vectors of a key
-// past the end, or in a block outside the pool, from here. Such a key's probability is 0, and
+// Zero bytes in global memory: the tile pass loads the key and value vectors of a key past the
+// end, or in a block outside the pool, from here. Such a key's probability is 0, and
 // 0 times whatever a pool row holds (inf or NaN included) would not be 0.
-static __device__ __align__(16) uint4 zero_vector = {0u, 0u, 0u, 0u};
+static __device__ __align__(32) uint4 zero_vector[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
 
 namespace pkv {
 namespace {
@@ -89,23 +89,10 @@ namespace {
 #ifndef PKV_ATTN_XCD_REMAP
 #define PKV_ATTN_XCD_REMAP 0
 #endif
-// Tile pass beside the row pass, float32 pools: 1 = key and value tiles go from HBM straight into
-// LDS (global_load_lds_dwordx4) through PKV_TILE_STAGES buffers, all but one in flight while one
-// is multiplied; 0 = through registers, one tile ahead. A tile pass on its own (one workgroup per
-// item) and the bfloat16 path always go through registers: the 96 KiB of stages allow one
-// workgroup per CU, where the register path runs three (measured: 0.86 vs 0.68 ms for config 3's
-// tiles alone; beside its row pass the direct path takes the call 1.56 -> 1.53 ms).
-#ifndef PKV_TILE_DMA
-#define PKV_TILE_DMA 1
-#endif
-// Direct-to-LDS path: LDS stages (2..5; 32 KiB each at head_dim 128: three leave room for two
-// row-pass workgroups on the CU).
-#ifndef PKV_TILE_STAGES
-#define PKV_TILE_STAGES 3
-#endif
-// Register path at head_dim 128: the occupancy target in waves per SIMD (its VGPR budget).
-// Measured on config 3's tiles alone: 3 waves (168 VGPRs) 0.68-0.70 ms, 2 waves (190 VGPRs,
-// value reads double-buffered) 0.73 ms.
+// The tile pass at head_dim 128: the occupancy target in waves per SIMD (its VGPR budget), for
+// bfloat16 pools and the float32 products. Measured on 8 chunks of 512 rows alone, bfloat16: 3
+// waves 0.235 ms, 2 waves 0.253 ms. The split float32 tiles take 237 VGPRs, two waves: held to
+// 168 they spill (0.53 against 0.62 ms, before their products were interleaved).
 #ifndef PKV_TILE_REG_WAVES
 #define PKV_TILE_REG_WAVES 3
 #endif
@@ -117,8 +104,6 @@ constexpr int kDefaultPartition = 512;
 constexpr int kTableSlots = kMaxPartition + 4;  // ceil(P / B) + 1 entries at most
 constexpr int kTileRows = 64;           // query rows per tile_partial workgroup (4 x 16)
 constexpr int kTileThreads = 256;
-constexpr int kTileStages = PKV_TILE_STAGES;  // LDS key/value stages of the direct-to-LDS path
-static_assert(kTileStages >= 2 && kTileStages <= 5, "2..5 direct-to-LDS stages");
 constexpr int kTileWhole = PKV_TILE_WHOLE;  // tile end partition: every key in one workgroup
 constexpr int kReduceThreads = 256;
 
@@ -315,9 +300,9 @@ __device__ __forceinline__ int block_of(int pos, const Params& a) {
 
 // Stage table entries of blocks [b0, b0 + nb) of sequence `seq` into LDS.
 __device__ __forceinline__ void stage_table(int* s_table, const Params& a, int seq, int b0, int nb,
-                                            int threads) {
+                                            int threads, int tid) {
   const int32_t* table = a.tables + static_cast<int64_t>(seq) * a.table_stride + b0;
-  for (int i = threadIdx.x; i < nb; i += threads) s_table[i] = table[i];
+  for (int i = tid; i < nb; i += threads) s_table[i] = table[i];
 }
 
 // Write one query row's partition result: final output (row r of out) when the row fits one
@@ -386,7 +371,7 @@ __global__ __launch_bounds__(kThreads) void row_partial_kernel(const Params a) {
 
   const int b0 = block_of<kPow2Block>(kbeg, a);
   const int nb = kend > kbeg ? block_of<kPow2Block>(kend - 1, a) - b0 + 1 : 0;
-  if (nb > 0) stage_table(s_table, a, seq, b0, nb, kThreads);
+  if (nb > 0) stage_table(s_table, a, seq, b0, nb, kThreads, threadIdx.x);
   __syncthreads();
 
   const int lane = threadIdx.x & (kWave - 1);
@@ -648,7 +633,7 @@ __global__ __launch_bounds__(kThreads) void row_partial_kernel(const Params a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Pass 2: tile_partial (fp32 MFMA). Lane l of a wavefront is (c = l / 16, n = l % 16); wavefront
+// Pass 2: tile_partial. With float32 products (tile_item): lane l of a wavefront is (c = l / 16, n = l % 16); wavefront
 // w owns the tile's queries 16w .. 16w + 15. Keys are staged in LDS kKeys at a time, as kSub
 // column blocks of 16 keys.
 //
@@ -692,36 +677,6 @@ __device__ __forceinline__ float column_sum(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// One 16-byte global load per lane written straight into LDS (global_load_lds_dwordx4): lane l
-// of the wavefront writes LDS bytes [lds + 16 l, lds + 16 l + 16). `lds` is the wavefront-uniform
-// LDS byte address, which the instruction takes in M0, set in the same statement (with the one
-// wait state GFX9 requires between an SALU write of M0 and an LDS DMA). The compiler does not
-// see these loads, so their completion is waited for explicitly (wait_vmcnt) before the barrier
-// that publishes the data.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_to_lds16(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// s_waitcnt vmcnt(N), leaving the other counters alone (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-// A workgroup barrier that orders LDS accesses only: unlike __syncthreads it does not wait for
-// outstanding global loads, so loads into the other LDS stages stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <int D>
 struct TileShape {
   static constexpr int kKeys = D <= 128 ? 32 : 16;  // keys per LDS tile (registers bound D = 256)
@@ -735,20 +690,7 @@ struct TileShape {
   // tiles in lane (c, n) are the kW adjacent output dims 16 kW g + kW (4 c + r) + [0, kW).
   static constexpr int kW = kNb >= 4 ? 4 : kNb;
   static constexpr int kGroups = kNb / kW;
-  // Direct-to-LDS stages: unpadded rows of D floats whose 16-byte chunks are XOR-swizzled by
-  // (row & 7): chunk q of key row r sits at chunk q ^ (r & 7). The S^T reads (16 rows, one
-  // chunk each) and the PV reads (4 rows, 16 adjacent chunks each) then spread over all LDS
-  // banks, as the padded rows do, while every 16-byte chunk stays whole for the DMA.
-  static constexpr int kChunks = kKeys * D / 4;            // 16-byte chunks of one K (or V) tile
-  static constexpr int kTileFloats = kKeys * D;
-  static constexpr int kStageFloats = 2 * kTileFloats;     // K tile then V tile
 };
-
-// LDS float offset of element `col` of key row `row` in a swizzled direct-to-LDS tile.
-template <int D>
-__device__ __forceinline__ int swz(int row, int col) {
-  return row * D + ((((col >> 2) ^ (row & 7))) << 2) + (col & 3);
-}
 
 // kW adjacent floats, the unit of one value-operand read and one output store of the tile pass.
 template <int W>
@@ -777,8 +719,8 @@ __device__ __forceinline__ void store_out_row(float* dst, const floatx4 (&o)[D /
 // come first). Every thread of the workgroup calls it with the same item; it returns early
 // (uniformly) for items outside the tile's partitions.
 template <typename KVT, int D, bool kPow2Block>
-__device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_table, float* s_k,
-                                          float* s_v, int* s_vis) {
+__device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, uint32_t tid, int* s_table,
+                                          float* s_k, float* s_v, int* s_vis) {
   static_assert(D % 16 == 0 && D >= 32, "the MFMA tile needs whole 16-wide output tiles");
   using S = TileShape<D>;
   constexpr int kKeys = S::kKeys;
@@ -803,10 +745,10 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_
   const int nrows = static_cast<int>(min<int64_t>(min(entry[1], kTileRows), a.num_queries - t0));
   const int seq = a.q_seq[t0];
 
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  if (threadIdx.x < kTileRows) {
-    s_vis[threadIdx.x] = static_cast<int>(threadIdx.x) < nrows ? row_visible(a, t0 + threadIdx.x) : 0;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if (tid < kTileRows) {
+    s_vis[tid] = static_cast<int>(tid) < nrows ? row_visible(a, t0 + tid) : 0;
   }
   __syncthreads();
   // The tile's longest visible row bounds its partitions (every wavefront reads all 64 entries).
@@ -824,7 +766,7 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_
   int b0 = block_of<kPow2Block>(kbeg, a);
   auto stage_window = [&]() {
     const int nb = min(last_block - b0 + 1, kTableSlots);
-    if (nb > 0) stage_table(s_table, a, seq, b0, nb, kTileThreads);
+    if (nb > 0) stage_table(s_table, a, seq, b0, nb, kTileThreads, tid);
   };
   stage_window();
 
@@ -944,7 +886,7 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_
     // table entry is read at a clamped index and not used).
 #pragma unroll
     for (int u = 0; u < kPerThread; ++u) {
-      const int v = threadIdx.x + u * kTileThreads;
+      const int v = tid + u * kTileThreads;
       const int row = v / kVecPerRow;
       const int col = (v - row * kVecPerRow) * kEpv;
       const int kpos = k0 + row;
@@ -977,7 +919,7 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_
     // Widen the prefetched tile (zeros for keys past kend or outside the pool) into LDS as float32.
 #pragma unroll
     for (int u = 0; u < kPerThread; ++u) {
-      const int v = threadIdx.x + u * kTileThreads;
+      const int v = tid + u * kTileThreads;
       if (v < kVecs) {
         const int row = v / kVecPerRow;
         const int col = (v - row * kVecPerRow) * kEpv;
@@ -1060,26 +1002,84 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, int* s_
   }
 }
 
-// One work item of the tile pass beside the row pass, float32 pools: the same item as tile_item,
-// with the key and value tiles moved from HBM straight into LDS (global_load_lds_dwordx4)
-// through kTileStages buffers, all but one in flight while one is multiplied, so no register
-// holds a tile on its way. In every step a wavefront whose rows all end before the step's first
-// key skips both products: its keys would all be masked (every score -inf, every probability
-// 0), so its registers would not change.
-template <int D, bool kPow2Block>
-__device__ __forceinline__ void tile_item_dma(const Params& a, uint32_t bid, int* s_table, float* s_kv,
-                                              int* s_vis) {
-  static_assert(D % 16 == 0 && D >= 32, "the MFMA tile needs whole 16-wide output tiles");
-  using S = TileShape<D>;
+// ---------------------------------------------------------------------------------------------
+// Tile items on bf16 MFMA with exact three-way splits. A float32 x is hi + mid + lo, each the next
+// 8 significant bits of x as a bfloat16 (truncated, so hi never overflows and the sum is exactly x
+// down to the subnormals); a product of two bfloat16 values is exact in float32 and the matrix
+// core accumulates in float32. With bfloat16 pools K and V are one piece, so an exact q * k or
+// p * v takes 3 products; with float32 pools the 6 products of weight >= 2^-16 are kept (the
+// dropped ones are below 2^-23 of the product). v_mfma_f32_16x16x32_bf16 does 16 times the work of
+// v_mfma_f32_16x16x4f32 per cycle, so the products cost 3/16 or 6/16 of the float32 ones.
+// ---------------------------------------------------------------------------------------------
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+
+// The next piece of two floats, packed as a bfloat16 pair (x0 in the low half); x0 and x1 become
+// what is left of them.
+__device__ __forceinline__ uint32_t take_piece(float& x0, float& x1) {
+  const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+  x0 -= __uint_as_float(u0 & 0xffff0000u);
+  x1 -= __uint_as_float(u1 & 0xffff0000u);
+  return __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+}
+__device__ __forceinline__ uint32_t last_piece(float x0, float x1) {
+  return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+}
+// Pins the computation of x to its place in the source (among instructions that are themselves
+// pinned); no instruction.
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+// Four keys' values of one dimension per lane (ds_read_b64_tr_b16): in each group of 16 lanes,
+// lane i reads 8 bytes of row i / 4 and receives column i of the 4 x 16 block.
+__device__ __forceinline__ short4v read_transposed(const uint16_t* p) {
+  typedef __attribute__((address_space(3))) short4v* lds_ptr;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+}
+
+template <typename KVT, int D>
+struct SplitShape {
+  static constexpr int kKeys = 32;  // the depth of one product over keys
+  static constexpr int kPlanes = std::is_same_v<KVT, float> ? 3 : 1;
+  static constexpr int kChunks = D / 8;  // 16-byte chunks of a bfloat16 row
+  // Padded LDS rows (elements): the 16 rows of a K read (one chunk each) and the 4 rows of a V
+  // read (32 bytes each) start in different banks, and every operand is a constant away from one
+  // address per lane. (Rows swizzled by chunk have no bank conflict left, against 12% of the
+  // cycles here, and measured the same in float32; in bfloat16 their addresses spill.)
+  static constexpr int kKRow = D + 8;
+  static constexpr int kVRow = D + (D % 128 == 0 ? 16 : D % 64 == 0 ? 48 : 16);
+  static constexpr int kKTile = kKeys * kKRow;  // one plane
+  static constexpr int kVTile = kKeys * kVRow;
+  static constexpr int kElems = kPlanes * (kKTile + kVTile);  // K planes, then V planes  // K planes, then V planes
+};
+
+// One work item of the tile pass (numbered as tile_item's). Returns true, with nothing written,
+// when a row's result is not finite: an infinity or NaN in the inputs does not survive the split
+// (inf - inf, 0 * inf), so the caller then computes the item with the float32 products of
+// tile_item.
+//
+// Bound: issue slots and power. Per 32 keys a wavefront issues 48 (bfloat16) or 96 products of 16
+// cycles and 200 or 365 vector instructions of 4, and the SIMD issues one of either per 4 cycles;
+// products and vector work overlap only where one wavefront alternates them (16 products and 32
+// vector instructions: 139 ns alternating, 125 ns for the products alone, 182 ns in two
+// wavefronts with 64), which the pinned order below is for. Measured on MI355X, 8 chunks of 512
+// rows at offsets up to 2048, 32 x 128 heads (86 GFLOP), same boxes: bfloat16 pools 0.685 ms with
+// float32 products, 0.250 with these unordered, 0.235 ordered; float32 pools 0.70, 0.505 and
+// 0.49; one chunk of 301 rows with 16 x 64 heads 29.6, 26.1 and 21.6 us. Relative error against
+// float64: 4.9e-7 (bfloat16) and 6.9e-7, 7.7e-7 with the float32 products, whose longer chains of
+// 4-term sums round more often.
+template <typename KVT, int D, bool kPow2Block>
+__device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, uint32_t tid, int* s_table,
+                                                uint16_t* s_kv, int* s_vis) {
+  using S = SplitShape<KVT, D>;
   constexpr int kKeys = S::kKeys;
-  constexpr int kSub = S::kSub;
-  constexpr int kD4 = S::kD4;
-  constexpr int kNb = S::kNb;
-  constexpr int kPer = S::kChunks / kTileThreads;  // DMA loads per lane per K (or V) tile
-  static_assert(kPer >= 1 && S::kChunks % kTileThreads == 0, "whole wavefront DMA loads per tile");
-  constexpr int kCpr = D / 4;  // 16-byte chunks per key row
-  constexpr int kAhead = kTileStages - 1;
-  constexpr int kVw = S::kW;  // output tile kVw g + e holds dims 16 kVw g + kVw i + e
+  constexpr int kPlanes = S::kPlanes;
+  constexpr int kSteps = D / 32;  // products over the head dimension
+  constexpr int kNb = D / 16;     // 16-dimension output blocks
+  constexpr bool kF32 = kPlanes == 3;
 
   const int h = static_cast<int>(bid % static_cast<uint32_t>(a.num_heads));
   const uint32_t rest = bid / static_cast<uint32_t>(a.num_heads);
@@ -1087,338 +1087,487 @@ __device__ __forceinline__ void tile_item_dma(const Params& a, uint32_t bid, int
   const int p = static_cast<int>(rest / static_cast<uint32_t>(a.num_tiles));
   const int32_t* entry = a.tiles + 4 * tile;
   const int64_t t0 = entry[0];
-  if (t0 < 0 || t0 >= a.num_queries) return;  // a tile outside the batch is skipped
-  // A whole tile is computed by its partition-0 workgroup alone, over every visible key.
+  if (t0 < 0 || t0 >= a.num_queries) return false;  // a tile outside the batch is skipped
   const bool whole = entry[3] == kTileWhole;
-  if (whole ? p != 0 : (p < entry[2] || (entry[3] > entry[2] && p >= entry[3]))) return;
+  if (whole ? p != 0 : (p < entry[2] || (entry[3] > entry[2] && p >= entry[3]))) return false;
   const int nrows = static_cast<int>(min<int64_t>(min(entry[1], kTileRows), a.num_queries - t0));
   const int seq = a.q_seq[t0];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  if (threadIdx.x < kTileRows) {
-    s_vis[threadIdx.x] = static_cast<int>(threadIdx.x) < nrows ? row_visible(a, t0 + threadIdx.x) : 0;
+
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if (tid < kTileRows) {
+    s_vis[tid] = static_cast<int>(tid) < nrows ? row_visible(a, t0 + tid) : 0;
   }
   __syncthreads();
-  // The tile's longest visible row bounds its partitions (every wavefront reads all 64 entries).
   int tile_vis = s_vis[lane];
 #pragma unroll
   for (int mask = 32; mask > 0; mask >>= 1) tile_vis = max(tile_vis, __shfl_xor(tile_vis, mask));
-  tile_vis = __builtin_amdgcn_readfirstlane(tile_vis);  // the same in every lane: keep it scalar
-  if (!whole && p >= parts_of(tile_vis, a.part_size)) return;
-  const int s_beg = whole ? 0 : p * a.part_size;
-  const int s_end = whole ? tile_vis : min(s_beg + a.part_size, tile_vis);
-
-  const float* kcache = static_cast<const float*>(a.kcache);
-  const float* vcache = static_cast<const float*>(a.vcache);
-  const int64_t head_off = static_cast<int64_t>(h) * D;
-  const int64_t row_stride = static_cast<int64_t>(a.num_heads) * D;
-  const uint32_t lds_kv = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_kv));
-  // Branch-free address arithmetic (selects, no divergent branches). A block's elements and a
-  // token row's fit 31 bits (launch_tiles takes this path only when block_size * num_heads *
-  // head_dim does).
-  const uint64_t block_elems = static_cast<uint64_t>(a.block_size) * static_cast<uint64_t>(row_stride);
-  const uint32_t row_elems = static_cast<uint32_t>(row_stride);
-  const uint32_t pool_blocks = static_cast<uint32_t>(min<int64_t>(a.num_blocks, INT32_MAX));
-  const int c = lane >> 4;
-  const int n = lane & 15;
-  const int qi = wave * 16 + n;  // this lane's query in the S^T layout
-
-  // The table entries of blocks [b0, b0 + kTableSlots) are staged in LDS. A partition always
-  // fits; a whole tile moves the window forward when the next key tile would leave it.
-  const int last_block = s_end > s_beg ? block_of<kPow2Block>(s_end - 1, a) : -1;
-  int b0 = block_of<kPow2Block>(s_beg, a);
+  tile_vis = __builtin_amdgcn_readfirstlane(tile_vis);
+  if (!whole && p >= parts_of(tile_vis, a.part_size)) return false;
+  const int kbeg = whole ? 0 : p * a.part_size;
+  const int kend = whole ? tile_vis : min(kbeg + a.part_size, tile_vis);
+  const int last_block = kend > kbeg ? block_of<kPow2Block>(kend - 1, a) : -1;
+  int b0 = block_of<kPow2Block>(kbeg, a);
   auto stage_window = [&]() {
     const int nb = min(last_block - b0 + 1, kTableSlots);
-    if (nb > 0) stage_table(s_table, a, seq, b0, nb, kTileThreads);
+    if (nb > 0) stage_table(s_table, a, seq, b0, nb, kTileThreads, tid);
   };
   stage_window();
 
+  const int c = lane >> 4;
+  const int n = lane & 15;
+  const int qi = wave * 16 + n;  // this lane's query
   const int my_vis = s_vis[qi];
   const bool q_ok = qi < nrows;
-  // This lane's row of queries and out (-1: a caller row outside the batch, skipped).
   const int io = static_cast<int>(io_row(a, t0 + (q_ok ? qi : 0)));
-  float qreg[kD4];
+
+  // The query's pieces: step s holds dimensions 32 s + 8 c .. + 7.
+  uint4v qp[3][kSteps];
   {
-    // Lanes past the tile read row t0 (always in the batch) and drop it, so every load is
-    // unconditional and the loads of a lane can all be in flight together.
     const float* qrow =
-        a.queries + static_cast<int64_t>(io < 0 ? 0 : io) * a.q_stride + static_cast<int64_t>(h) * D + c * kD4;
-    float raw[kD4];
+        a.queries + static_cast<int64_t>(io < 0 ? 0 : io) * a.q_stride + static_cast<int64_t>(h) * D + 8 * c;
 #pragma unroll
-    for (int i = 0; i < kD4; ++i) raw[i] = qrow[i];
+    for (int s = 0; s < kSteps; ++s) {
+      float raw[8];
 #pragma unroll
-    for (int i = 0; i < kD4; ++i) qreg[i] = q_ok ? raw[i] * a.scale_log2 : 0.f;
+      for (int e = 0; e < 8; ++e) raw[e] = qrow[32 * s + e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) raw[e] = q_ok ? raw[e] * a.scale_log2 : 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        qp[0][s][e] = take_piece(raw[2 * e], raw[2 * e + 1]);
+        qp[1][s][e] = take_piece(raw[2 * e], raw[2 * e + 1]);
+        qp[2][s][e] = last_piece(raw[2 * e], raw[2 * e + 1]);
+      }
+    }
   }
+
   floatx4 o[kNb];
 #pragma unroll
   for (int b = 0; b < kNb; ++b) o[b] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float m_ref = -INFINITY;  // the same in the four lanes of a query
-  float l_part = 0.f;       // this lane's share of the query's sum
-  const int lim = min(my_vis, s_end);
-  int wave_lim = lim;  // the wavefront's last key + 1: steps from there on are all masked
+  float m_ref = -INFINITY;
+  float l_part = 0.f;
+
+  const KVT* kcache = static_cast<const KVT*>(a.kcache);
+  const KVT* vcache = static_cast<const KVT*>(a.vcache);
+  const int64_t head_off = static_cast<int64_t>(h) * D;
+  const int64_t row_stride = static_cast<int64_t>(a.num_heads) * D;
+  __syncthreads();  // s_table ready
+
+  const int lim = min(my_vis, kend);
+  int wave_lim = lim;
 #pragma unroll
   for (int mask = 32; mask > 0; mask >>= 1) wave_lim = max(wave_lim, __shfl_xor(wave_lim, mask));
   wave_lim = __builtin_amdgcn_readfirstlane(wave_lim);
-  // Every row of the wavefront sees the keys below wave_full: a key tile that ends by then, with
-  // every key in a block inside the pool (all bits of its key mask set), needs no per-key mask.
   int wave_full = q_ok ? lim : INT32_MAX;
 #pragma unroll
   for (int mask = 32; mask > 0; mask >>= 1) wave_full = min(wave_full, __shfl_xor(wave_full, mask));
   wave_full = __builtin_amdgcn_readfirstlane(wave_full);
-  constexpr uint32_t kAllKeys = static_cast<uint32_t>((uint64_t{1} << kKeys) - 1u);
-  __syncthreads();  // s_table ready
 
-  // Table entry of key kpos (clamped into the window; callers discard it when kpos is out).
-  auto table_at = [&](int kpos) {
-    const int lb = min(max(block_of<kPow2Block>(kpos, a) - b0, 0), kTableSlots - 1);
-    return s_table[lb];
+  // A thread moves chunks of 8 elements of a key (value) row: one 16-byte vector of a bfloat16 row,
+  // two of a float32 row.
+  constexpr int kVecs = kKeys * S::kChunks;
+  constexpr int kPer = (kVecs + kTileThreads - 1) / kTileThreads;
+  constexpr int kLoads = kF32 ? 2 : 1;
+  const bool moves = kVecs % kTileThreads == 0 || tid < kVecs;
+  const uint32_t my_row = tid / S::kChunks;  // chunk u is in row my_row + u * kRowStep
+  constexpr uint32_t kRowStep = kTileThreads / S::kChunks;
+  const uint32_t my_col = tid % S::kChunks * 8;
+  const uint64_t row_bytes = static_cast<uint64_t>(row_stride) * sizeof(KVT);
+  const char* kbase = reinterpret_cast<const char*>(kcache + head_off + my_col);
+  const char* vbase = reinterpret_cast<const char*>(vcache + head_off + my_col);
+  const uint32_t pool_blocks = static_cast<uint32_t>(min<int64_t>(a.num_blocks, INT32_MAX));
+  uint16_t* sk = s_kv;
+  uint16_t* sv = s_kv + kPlanes * S::kKTile;
+  uint16_t* k_put = sk + my_row * S::kKRow + my_col;
+  uint16_t* v_put = sv + my_row * S::kVRow + my_col;
+  const uint16_t* k_get = sk + n * S::kKRow + 8 * c;
+  const uint16_t* v_get = sv + (4 * c + (n >> 2)) * S::kVRow + 4 * (n & 3);
+
+  // Where key tile i is: the token row of each of this thread's chunks (ok: a key before kend in a
+  // block inside the pool), and its key mask (bit k: key k of the tile is ok).
+  struct Where {
+    int entry[kPer];
+    uint32_t slot[kPer];
+    bool ok[kPer];
+    int mask_entry;
+    uint32_t mask;
   };
-  // Element offsets of this lane's kPer chunks of key tile k0 (bit u of `valid`: chunk u's key
-  // is before the end and in the pool), and the tile's key mask.
-  auto prepare = [&](int k0, int lane_v, int64_t (&off)[kPer], uint32_t& valid) -> uint32_t {
-    valid = 0u;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int chunk = (wave * kPer + u) * kWave + lane_v;
-      const int row = chunk / kCpr;
-      const int col = ((chunk % kCpr) ^ (row & 7)) * 4;
-      const int kpos = k0 + row;
-      const int blk = table_at(kpos);
-      const bool ok = (kpos < s_end) & (static_cast<uint32_t>(blk) < pool_blocks);
-      const uint32_t within = kPow2Block ? (kpos & (a.block_size - 1)) : kpos % a.block_size;
-      const uint32_t blk_u = ok ? static_cast<uint32_t>(blk) : 0u;
-      const uint32_t row_off = ok ? within * row_elems : 0u;
-      off[u] = static_cast<int64_t>(blk_u * block_elems) + static_cast<int64_t>(row_off) + head_off + col;
-      valid |= ok ? 1u << u : 0u;
+  auto entry_at = [&](int kpos) {
+    return s_table[min(max(block_of<kPow2Block>(kpos, a) - b0, 0), kTableSlots - 1)];
+  };
+  auto locate_read = [&](Where& w, int i, int u) {  // u == kPer: the mask's key
+    const int kpos = kbeg + i * kKeys + (u < kPer ? static_cast<int>(my_row + u * kRowStep) : lane);
+    if (u < kPer) {
+      w.entry[u] = entry_at(kpos);
+    } else {
+      w.mask_entry = entry_at(kpos);
     }
-    const int kpos = k0 + lane_v;
-    const bool ok = (lane_v < kKeys) & (kpos < s_end) &
-                    (static_cast<uint32_t>(table_at(kpos)) < pool_blocks);
-    return static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(ok));
   };
-  // Queue the chunks' loads into stage `buf`; an invalid chunk loads zero_vector.
-  auto fire = [&](int buf, const int64_t (&off)[kPer], uint32_t valid) {
-    const uint32_t dst = lds_kv + static_cast<uint32_t>(buf * S::kStageFloats * 4 + wave * kPer * 1024);
-    const float* zero = reinterpret_cast<const float*>(&zero_vector);
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const bool ok = (valid >> u) & 1u;
-      load_to_lds16(ok ? kcache + off[u] : zero, dst + u * 1024);
-      load_to_lds16(ok ? vcache + off[u] : zero, dst + u * 1024 + S::kTileFloats * 4);
+  auto locate_slot = [&](Where& w, int i, int u) {
+    const int kpos = kbeg + i * kKeys + (u < kPer ? static_cast<int>(my_row + u * kRowStep) : lane);
+    if (u < kPer) {
+      w.ok[u] = (kpos < kend) & (static_cast<uint32_t>(w.entry[u]) < pool_blocks);
+      const uint32_t within = kPow2Block ? kpos & (a.block_size - 1) : kpos % a.block_size;
+      w.slot[u] = static_cast<uint32_t>(w.entry[u]) * static_cast<uint32_t>(a.block_size) + within;
+    } else {
+      const bool ok = (lane < kKeys) & (kpos < kend) & (static_cast<uint32_t>(w.mask_entry) < pool_blocks);
+      w.mask = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(ok));
     }
   };
-  // One key tile's scores st -> probabilities pr, updating the running reference and sum. A
-  // key counts when it is below the lane's limit and its bit in kmask is set. The rescale is
-  // branch-free (alpha is exactly 1 in lanes that keep their reference), so the step stays
-  // one block of straight-line code the compiler can interleave.
-  auto softmax_step = [&](floatx4 (&st)[kSub], int k0, uint32_t kmask, float (&pr)[kSub][4]) {
-    float sc[kSub][4];
-    float mx = -INFINITY;
-    if (k0 + kKeys <= wave_full && kmask == kAllKeys) {  // wavefront-uniform: nothing masked
+  auto locate = [&](int i) {
+    Where w;
 #pragma unroll
-      for (int j = 0; j < kSub; ++j) {
+    for (int u = 0; u <= kPer; ++u) locate_read(w, i, u);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          sc[j][r] = st[j][r];
-          mx = fmaxf(mx, sc[j][r]);
+    for (int u = 0; u <= kPer; ++u) locate_slot(w, i, u);
+    return w;
+  };
+  auto load = [&](uint4v (&raw)[kPer][kLoads], const char* base, const Where& w, int u) {
+    const char* at = w.ok[u] ? base + w.slot[u] * row_bytes : reinterpret_cast<const char*>(zero_vector);
+#pragma unroll
+    for (int x = 0; x < kLoads; ++x) raw[u][x] = reinterpret_cast<const uint4v*>(at)[x];
+  };
+  auto load_all = [&](uint4v (&raw)[kPer][kLoads], const char* base, const Where& w) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) load(raw, base, w, u);
+  };
+  // Staging of a chunk into its planes, `plane` elements apart, in kPutTasks steps per chunk: one
+  // piece of one pair each (float32), then the LDS writes.
+  constexpr int kPutTasks = kF32 ? 9 : 1;
+  uint4v pl[3];
+  auto put = [&](uint16_t* at, int row, int plane, uint4v (&raw)[kPer][kLoads], int task) {
+    const int u = task / kPutTasks, step = task % kPutTasks;
+    if constexpr (kF32) {
+      if (step < 8) {
+        const int e = step / 2;  // pair of the chunk
+        float x0 = __uint_as_float(raw[u][e / 2][2 * (e % 2)]), x1 = __uint_as_float(raw[u][e / 2][2 * (e % 2) + 1]);
+        if (step % 2 == 0) {
+          uint32_t hi = take_piece(x0, x1);
+          pin(hi);
+          pl[0][e] = hi;
+          raw[u][e / 2][2 * (e % 2)] = __float_as_uint(x0);
+          raw[u][e / 2][2 * (e % 2) + 1] = __float_as_uint(x1);
+        } else {
+          uint32_t mid = take_piece(x0, x1);
+          uint32_t lo = last_piece(x0, x1);
+          pin(lo);
+          pl[1][e] = mid;
+          pl[2][e] = lo;
+        }
+      } else if (moves) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          *reinterpret_cast<uint4v*>(at + u * static_cast<int>(kRowStep) * row + q * plane) = pl[q];
         }
       }
-    } else {
+    } else if (moves) {
+      *reinterpret_cast<uint4v*>(at + u * static_cast<int>(kRowStep) * row) = raw[u][0];
+    }
+  };
+  auto put_all = [&](uint16_t* at, int row, int plane, uint4v (&raw)[kPer][kLoads]) {
 #pragma unroll
-      for (int j = 0; j < kSub; ++j) {
+    for (int t = 0; t < kPer * kPutTasks; ++t) put(at, row, plane, raw, t);
+  };
+
+  auto product = [](const uint4v& x, const uint4v& y, const floatx4& z) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), z,
+                                                   0, 0, 0);
+  };
+  // Product m of x * y from the pieces of y and of x (one piece: a bfloat16 pool), smallest first.
+  constexpr int kProducts = kF32 ? 6 : 3;
+  auto product_of = [&](int m, const uint4v (&x)[kPlanes], const uint4v& y0, const uint4v& y1, const uint4v& y2,
+                        const floatx4& z) {
+    if constexpr (kF32) {
+      constexpr int kX[6] = {2, 1, 0, 1, 0, 0};
+      constexpr int kY[6] = {0, 1, 2, 0, 1, 0};
+      return product(x[kX[m]], kY[m] == 0 ? y0 : kY[m] == 1 ? y1 : y2, z);
+    } else {
+      return product(x[0], m == 0 ? y2 : m == 1 ? y1 : y0, z);
+    }
+  };
+  // Runs `tasks` (vector work, numbered) spread among the products of kOps operand reads. The
+  // order is pinned: a wavefront's vector instructions run in the shadow of its own products only
+  // where they alternate, and operands are read one read ahead of their products.
+  constexpr int kAhead = 1;
+  auto run = [&](auto ops_tag, auto tasks_tag, auto&& read, auto&& multiply, auto&& task) {
+    constexpr int kOps = decltype(ops_tag)::value;
+    constexpr int kTasks = decltype(tasks_tag)::value;
+    constexpr int kSlots = kOps * kProducts;
+    uint4v x[kAhead + 1][kPlanes];
+#pragma unroll
+    for (int g = 0; g < kAhead && g < kOps; ++g) read(g, x[g]);
+    constexpr int kPerSlot = (kTasks + kSlots - 1) / kSlots;
+#pragma unroll
+    for (int g = 0; g < kOps; ++g) {
+      if (g + kAhead < kOps) read(g + kAhead, x[(g + kAhead) % (kAhead + 1)]);
+#pragma unroll
+      for (int m = 0; m < kProducts; ++m) {
+        multiply(g, m, x[g % (kAhead + 1)]);
+        const int slot = g * kProducts + m;
+        const int first = (slot * kTasks + kSlots - 1) / kSlots;
+#pragma unroll
+        for (int t = 0; t < kPerSlot; ++t) {
+          if (first + t < ((slot + 1) * kTasks + kSlots - 1) / kSlots) task(first + t);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // S^T of the key tile in LDS: register r of st[j] = S[query n][key 16 j + 4 c + r of the tile].
+  floatx4 st[2], next[2];
+  auto read_keys = [&](int g, uint4v (&x)[kPlanes]) {
+#pragma unroll
+    for (int q = 0; q < kPlanes; ++q) {
+      x[q] = *reinterpret_cast<const uint4v*>(k_get + (q * S::kKTile + 16 * (g & 1) * S::kKRow + 32 * (g >> 1)));
+    }
+  };
+  auto multiply_keys = [&](int g, int m, const uint4v (&x)[kPlanes]) {
+    const int s = g >> 1;
+    next[g & 1] = product_of(m, x, qp[0][s], qp[1][s], qp[2][s], s == 0 && m == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : next[g & 1]);
+  };
+  // O^T += V^T P^T: register r of o[b] = O[query n][16 b + 4 c + r].
+  uint4v pp[3];
+  auto read_values = [&](int b, uint4v (&x)[kPlanes]) {
+#pragma unroll
+    for (int q = 0; q < kPlanes; ++q) {
+      const uint16_t* plane = v_get + (q * S::kVTile + 16 * b);
+      const auto lo4 = __builtin_bit_cast(uint2, read_transposed(plane));
+      const auto hi4 = __builtin_bit_cast(uint2, read_transposed(plane + 16 * S::kVRow));
+      x[q] = uint4v{lo4.x, lo4.y, hi4.x, hi4.y};
+    }
+  };
+  auto multiply_values = [&](int b, int m, const uint4v (&x)[kPlanes]) {
+    o[b] = product_of(m, x, pp[0], pp[1], pp[2], o[b]);
+  };
+  // Masks tile i's scores and raises the reference when one passes it by more than kLazyLog2.
+  auto raise_reference = [&](int i, uint32_t mask) {
+    const int k0 = kbeg + i * kKeys;
+    if (k0 + kKeys > wave_full || mask != 0xffffffffu) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kk = 16 * j + 4 * c + r;
-          sc[j][r] = (k0 + kk) < lim && ((kmask >> kk) & 1u) ? st[j][r] : -INFINITY;
-          mx = fmaxf(mx, sc[j][r]);
+          st[j][r] = (k0 + kk) < lim && ((mask >> kk) & 1u) ? st[j][r] : -INFINITY;
         }
       }
     }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[j][r]);
+    }
     mx = column_max(mx);
-    // Raise the reference only when a score passes it by more than kLazyLog2 (or it is unset).
     const bool raise = mx > m_ref + kLazyLog2 || (m_ref == -INFINITY && mx > -INFINITY);
-    const float m_next = raise ? mx : m_ref;
-    const float alpha = raise ? fast_exp2(m_ref - m_next) : 1.f;  // exp2(-inf) = 0
-    l_part *= alpha;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      const float m_next = raise ? mx : m_ref;
+      const float alpha = raise ? fast_exp2(m_ref - m_next) : 1.f;
+      l_part *= alpha;
 #pragma unroll
-    for (int b = 0; b < kNb; ++b) o[b] *= alpha;
-    m_ref = m_next;
-    const float shift = m_ref == -INFINITY ? 0.f : m_ref;
-#pragma unroll
-    for (int j = 0; j < kSub; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pr[j][r] = fast_exp2(sc[j][r] - shift);
-        l_part += pr[j][r];
-      }
+      for (int b = 0; b < kNb; ++b) o[b] *= alpha;
+      m_ref = m_next;
+    }
+  };
+  // This lane's probabilities in pieces, the B operand whose 8 keys are 4 c + [0, 4) of both
+  // blocks: kProbTasks steps, three per pair.
+  constexpr int kProbTasks = 12;
+  float p0, p1;
+  auto probability = [&](int task) {
+    const int e = task / 3;  // pair
+    if (task % 3 == 0) {
+      const float shift = m_ref == -INFINITY ? 0.f : m_ref;
+      p0 = fast_exp2(st[e / 2][2 * (e % 2)] - shift);
+      p1 = fast_exp2(st[e / 2][2 * (e % 2) + 1] - shift);
+      l_part += p0;
+      l_part += p1;
+      pin(l_part);
+    } else if (task % 3 == 1) {
+      uint32_t hi = take_piece(p0, p1);
+      pin(hi);
+      pp[0][e] = hi;
+    } else {
+      uint32_t mid = take_piece(p0, p1);
+      uint32_t lo = last_piece(p0, p1);
+      pin(lo);
+      pp[1][e] = mid;
+      pp[2][e] = lo;
     }
   };
 
-  // The pipeline: step i waits for its own loads (vmcnt), then one barrier publishes every
-  // wavefront's share and also closes step i - 1, whose buffer the loads of step
-  // i + kTileStages - 1 then fill. Those are queued between the step's two products. Every
-  // lane issues the same loads in every step, past the last step too: a lane whose key is past
-  // the end or in a block outside the pool loads zero_vector instead, and the key's bit in the
-  // step's mask stays clear.
-  const int nsteps = s_end > s_beg ? (s_end - s_beg + kKeys - 1) / kKeys : 0;
-  uint32_t kmask[kAhead];  // key masks of steps i .. i + kAhead - 1
-  wait_vmcnt<0>();  // the query loads (and earlier stores) complete before the pipeline's loads
-  if (nsteps > 0) {
+  // The pipeline over key tiles i: the products of one tile run among the vector work of others.
+  //   A: the scores of tile i + 1 (its keys in LDS) among the probabilities of tile i and the
+  //      staging of its values, whose registers then take the loads of values i + 1; barrier
+  //   B: the output of tile i (its values in LDS) among the staging of the keys of tile i + 2,
+  //      whose registers then take the loads of keys i + 3; barrier
+  // Loads so have a whole step to arrive. A wavefront without rows only stages.
+  const int ntiles = (kend - kbeg + kKeys - 1) / kKeys;
+  const bool active = wave_lim > kbeg;
+  if (ntiles > 0) {
+    using std::integral_constant;
+    auto nothing = [](int) {};
+    uint4v kraw[kPer][kLoads];
+    uint4v vraw[kPer][kLoads];
+    Where w0 = locate(0);
+    Where w1 = locate(1);
+    Where w2 = locate(2);
+    uint32_t mask = w0.mask;
+    load_all(kraw, kbase, w0);
+    load_all(vraw, vbase, w0);
+    put_all(k_put, S::kKRow, S::kKTile, kraw);
+    load_all(kraw, kbase, w1);
+    __syncthreads();
+    if (active) run(integral_constant<int, 2 * kSteps>{}, integral_constant<int, 0>{}, read_keys, multiply_keys, nothing);
+    __syncthreads();
+    put_all(k_put, S::kKRow, S::kKTile, kraw);
+    load_all(kraw, kbase, w2);
+    __syncthreads();
+    // w1, w2: tiles i + 1 and i + 2. The table window follows tile i + 3, which B locates.
+    auto move_window = [&](int i) {
+      if (block_of<kPow2Block>(min(kbeg + (i + 4) * kKeys, kend) - 1, a) >= b0 + kTableSlots) {
+        b0 = block_of<kPow2Block>(kbeg + (i + 3) * kKeys, a);
+        stage_window();
+      }
+    };
+    constexpr int kPuts = kPer * kPutTasks;
+    if (active) {
+      int i = 0;
+      for (; i + 1 < ntiles; ++i) {
+        move_window(i);
+        st[0] = next[0];
+        st[1] = next[1];
+        raise_reference(i, mask);
+        __builtin_amdgcn_sched_barrier(0);
+        run(integral_constant<int, 2 * kSteps>{}, integral_constant<int, kProbTasks + kPuts + kPer>{}, read_keys,
+            multiply_keys, [&](int t) {
+              if (t < kProbTasks) {
+                probability(t);
+              } else if (t < kProbTasks + kPuts) {
+                put(v_put, S::kVRow, S::kVTile, vraw, t - kProbTasks);
+              } else {
+                load(vraw, vbase, w1, t - kProbTasks - kPuts);
+              }
+            });
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        mask = w1.mask;
+        w1 = w2;
+        run(integral_constant<int, kNb>{}, integral_constant<int, 2 * (kPer + 1) + kPuts + kPer>{}, read_values,
+            multiply_values, [&](int t) {
+              if (t <= kPer) {
+                locate_read(w2, i + 3, t);
+              } else if (t <= 2 * kPer + 1) {
+                locate_slot(w2, i + 3, t - kPer - 1);
+              } else if (t < 2 * kPer + 2 + kPuts) {
+                put(k_put, S::kKRow, S::kKTile, kraw, t - 2 * kPer - 2);
+              } else {
+                load(kraw, kbase, w2, t - 2 * kPer - 2 - kPuts);
+              }
+            });
+        __syncthreads();
+      }
+      st[0] = next[0];
+      st[1] = next[1];
+      raise_reference(i, mask);
+      put_all(v_put, S::kVRow, S::kVTile, vraw);
 #pragma unroll
-    for (int st = 0; st < kAhead; ++st) {
-      int64_t off[kPer];
-      uint32_t valid;
-      kmask[st] = prepare(s_beg + st * kKeys, lane, off, valid);
-      fire(st, off, valid);
-    }
-  }
-  int buf = 0;
-  for (int i = 0; i < nsteps; ++i) {
-    const int k0 = s_beg + i * kKeys;
-    wait_vmcnt<(kAhead - 1) * 2 * kPer>();  // this step's loads have landed
-    lds_barrier();
-    const int k_next = k0 + kAhead * kKeys;  // the tile whose loads this step queues
-    if (block_of<kPow2Block>(min(k_next + kKeys, s_end) - 1, a) >= b0 + kTableSlots) {
-      // A whole tile moves its table window; no wavefront reads the table between the barrier
-      // above and the one below.
-      b0 = block_of<kPow2Block>(k_next, a);
-      stage_window();
-      lds_barrier();
-    }
-    const bool work = k0 < wave_lim;  // wavefront-uniform
-    // The swizzled LDS addresses are lane constants; they are recomputed from an opaque copy
-    // of the lane index each step (a few VALU operations) instead of being hoisted out of the
-    // loop, which would hold about 20 more VGPRs and cost the CU a row-pass workgroup.
-    int lane_o = lane;
-    asm volatile("" : "+v"(lane_o));
-    const int cl = lane_o >> 4;
-    const int nl = lane_o & 15;
-    const float* sk = s_kv + buf * S::kStageFloats;
-    const float* sv = sk + S::kTileFloats;
-
-    // S^T blocks: register r of st[j] = S[query n][key k0 + 16j + 4c + r]. Lane (c, n) reads
-    // chunk c * kD4 / 4 + q of key row 16 j + n, swizzled by n & 7.
-    floatx4 st[kSub];
-#pragma unroll
-    for (int j = 0; j < kSub; ++j) st[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    if (work) {
-#pragma unroll
-      for (int q = 0; q < kD4 / 4; ++q) {
-#pragma unroll
-        for (int j = 0; j < kSub; ++j) {
-          const float4 kv = *reinterpret_cast<const float4*>(
-              sk + (16 * j + nl) * D + (((cl * (kD4 / 4) + q) ^ (nl & 7)) << 2));
-          st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qreg[4 * q], st[j], 0, 0, 0);
-          st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qreg[4 * q + 1], st[j], 0, 0, 0);
-          st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qreg[4 * q + 2], st[j], 0, 0, 0);
-          st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qreg[4 * q + 3], st[j], 0, 0, 0);
-        }
+      for (int t = 0; t < kProbTasks; ++t) probability(t);
+      __syncthreads();
+      run(integral_constant<int, kNb>{}, integral_constant<int, 0>{}, read_values, multiply_values, nothing);
+    } else {
+      for (int i = 0; i < ntiles; ++i) {
+        move_window(i);
+        put_all(v_put, S::kVRow, S::kVTile, vraw);
+        load_all(vraw, vbase, w1);
+        __syncthreads();
+        if (i + 1 == ntiles) break;
+        put_all(k_put, S::kKRow, S::kKTile, kraw);
+        w1 = w2;
+        w2 = locate(i + 3);
+        load_all(kraw, kbase, w2);
+        __syncthreads();
       }
     }
-    // Queue step i + kAhead's loads into the buffer step i - 1 used. Their address arithmetic
-    // is scheduled among the PV products below, not the S^T products above (which would keep
-    // more registers live across the S^T loop).
-    __builtin_amdgcn_sched_barrier(0);
-    uint32_t next_mask;
-    {
-      int64_t off[kPer];
-      uint32_t valid;
-      next_mask = prepare(k_next, lane_o, off, valid);
-      fire(buf == 0 ? kAhead : buf - 1, off, valid);
-    }
-    if (work) {
-      float pr[kSub][4];
-      softmax_step(st, k0, kmask[0], pr);
-      // O^T += V^T P^T. Lane (c, n) reads the kVw adjacent floats at column 16 kVw g + kVw n
-      // of row 16 j + 4 c + step: part of chunk 4 g + n (kVw = 4: the whole chunk) or
-      // g + n / 2 (kVw = 2), swizzled by (4 c + step) & 7, so each step needs one lane base and
-      // j and g are immediate offsets. The products are accumulated in the register path's
-      // order (j, then step, then output tile), so both paths round identically.
-#pragma unroll
-      for (int j = 0; j < kSub; ++j) {
-#pragma unroll
-        for (int step = 0; step < 4; ++step) {
-          const int swz_row = 4 * (cl & 1) + step;  // (16 j + 4 c + step) & 7
-          const int col = kVw * nl;
-          const float* vbase = sv + 4 * cl * D + ((((col >> 2) ^ swz_row)) << 2) + (col & 3);
-#pragma unroll
-          for (int g = 0; g < kNb / kVw; ++g) {
-            const floatw<kVw> x =
-                *reinterpret_cast<const floatw<kVw>*>(vbase + (16 * j + step) * D + 16 * kVw * g);
-#pragma unroll
-            for (int e = 0; e < kVw; ++e) {
-              const int b = kVw * g + e;
-              o[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], pr[j][step], o[b], 0, 0, 0);
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int st2 = 0; st2 + 1 < kAhead; ++st2) kmask[st2] = kmask[st2 + 1];
-    kmask[kAhead - 1] = next_mask;
-    buf = buf == kTileStages - 1 ? 0 : buf + 1;
   }
-  wait_vmcnt<0>();  // the loads queued past the last step land before the LDS is reused
 
-  // Epilogue: register r of tile kVw g + e is O[query n][16 kVw g + kVw (4c + r) + e].
   const float l = column_sum(l_part);
-  // A whole tile covered every visible key of its rows: their outputs are final.
+  float poison = l * 0.f;  // NaN once any value of the row is not finite
+#pragma unroll
+  for (int b = 0; b < kNb; ++b) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) poison = fmaf(o[b][r], 0.f, poison);
+  }
+  if (__syncthreads_or(poison != 0.f)) return true;
+  if (!q_ok) return false;
   const int row_parts = whole ? 1 : parts_of(my_vis, a.part_size);
-  if (!q_ok || p >= row_parts) return;
-  const int64_t qh = (t0 + qi) * a.num_heads + h;
+  if (p >= row_parts) return false;
+  float* dst;
+  float sum = 1.f;
   if (row_parts == 1) {
-    if (io >= 0) {
-      store_out_row<D, kVw>(a.out + (static_cast<int64_t>(io) * a.num_heads + h) * D, o, c, l > 0.f ? l : 1.f);
-    }
+    if (io < 0) return false;
+    dst = a.out + (static_cast<int64_t>(io) * a.num_heads + h) * D;
+    sum = l > 0.f ? l : 1.f;
   } else {
-    const int64_t slot = qh * a.max_parts + p;
-    store_out_row<D, kVw>(a.ws_acc + slot * D, o, c, 1.f);
+    const int64_t slot = ((t0 + qi) * a.num_heads + h) * a.max_parts + p;
+    dst = a.ws_acc + slot * D;
     if (c == 0) {
       a.ws_ml[2 * slot] = m_ref;
       a.ws_ml[2 * slot + 1] = l;
     }
   }
+#pragma unroll
+  for (int b = 0; b < kNb; ++b) {
+    const floatx4 x = {o[b][0] / sum, o[b][1] / sum, o[b][2] / sum, o[b][3] / sum};
+    *reinterpret_cast<floatx4*>(dst + 16 * b + 4 * c) = x;
+  }
+  return false;
+}
+
+enum class TilePath { kSplit, kFloat };
+
+template <typename KVT, int D>
+constexpr int tile_waves(TilePath path) {
+  if (D != 128) return 1;
+  return path == TilePath::kSplit && std::is_same_v<KVT, float> ? 2 : PKV_TILE_REG_WAVES;
 }
 
 // The tile pass: workgroup w computes items w, w + gridDim.x, ... of the num_items (tile,
 // partition, head) items. With one item per workgroup the grid is the item count; beside the
-// row pass the host launches one workgroup per CU instead, so the tile pass holds one wave per
-// SIMD and leaves the rest of each CU to the memory-bound row pass. The register path at
-// head_dim 128 is held to 168 VGPRs (three waves per SIMD; it needs about 170 unconstrained,
-// which allows two); the other instantiations have no occupancy target. Its wavefronts run at
+// row pass the host launches a few workgroups per CU instead (launch_tiles), which leaves the rest
+// of each CU to the memory-bound row pass. Its wavefronts run at
 // instruction-arbiter priority 1 (the row pass keeps 0): beside the row pass the tile items are
 // the ones that finish last, and the memory-bound row wavefronts lose little by yielding issue
 // slots (measured: the prefix-sharing step's call 0.2333-0.2369 -> 0.2311-0.2335 ms, the mixed
 // bfloat16 call 1.105-1.110 -> 1.102-1.107 ms; alone, where every wavefront is a tile's, it
 // changes nothing). The reverse, the row pass at priority 1, starves the tiles (the mixed
 // float32 call 1.48 -> 1.97 ms).
-template <typename KVT, int D, bool kPow2Block, bool kDma>
+template <typename KVT, int D, bool kPow2Block, TilePath kPath>
 __global__ __launch_bounds__(kTileThreads)
-__attribute__((amdgpu_waves_per_eu(!kDma && D == 128 ? PKV_TILE_REG_WAVES : 1)))
+__attribute__((amdgpu_waves_per_eu(tile_waves<KVT, D>(kPath))))
 void tile_partial_kernel(const Params a, uint32_t num_items) {
   using S = TileShape<D>;
   __builtin_amdgcn_s_setprio(1);
   __shared__ int s_table[kTableSlots];
   __shared__ int s_vis[kTileRows];
-  if constexpr (kDma) {
-    static_assert(std::is_same_v<KVT, float>, "the direct-to-LDS tiles are float32");
-    // The stages are dynamic LDS (kTileStages * S::kStageFloats floats, sized at launch). From
-    // a static array of their size the compiler would infer one wave per SIMD and reserve the
-    // registers of that occupancy (257 instead of the 152 used), which leaves room for one
-    // row-pass workgroup per CU instead of two.
-    extern __shared__ __align__(16) float s_kv[];
-    for (uint32_t item = blockIdx.x; item < num_items; item += gridDim.x) {
-      __syncthreads();  // the previous item's reads of LDS are done
-      tile_item_dma<D, kPow2Block>(a, item, s_table, s_kv, s_vis);
+  constexpr bool kSplit = kPath == TilePath::kSplit;
+  constexpr int kRows = S::kKeys * S::kRow;  // floats of a key (or value) tile of tile_item
+  constexpr int kSplitFloats = kSplit ? SplitShape<KVT, D>::kElems / 2 : 0;
+  __shared__ __align__(16) float s_kv[2 * kRows > kSplitFloats ? 2 * kRows : kSplitFloats];
+  for (uint32_t item = blockIdx.x; item < num_items; item += gridDim.x) {
+    __syncthreads();  // the previous item's reads of LDS are done
+    // An opaque thread index per item and path: values derived from it stay inside, where the
+    // compiler would otherwise keep both paths' lane constants in registers across the loop.
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    tid &= kTileThreads - 1;
+    if constexpr (kSplit) {
+      if (!tile_item_split<KVT, D, kPow2Block>(a, item, tid, s_table, reinterpret_cast<uint16_t*>(s_kv), s_vis)) {
+        continue;
+      }
+      asm volatile("" : "+v"(tid));
     }
-  } else {
-    __shared__ float s_k[S::kKeys * S::kRow];
-    __shared__ float s_v[S::kKeys * S::kRow];
-    for (uint32_t item = blockIdx.x; item < num_items; item += gridDim.x) {
-      __syncthreads();  // the previous item's reads of LDS are done
-      tile_item<KVT, D, kPow2Block>(a, item, s_table, s_k, s_v, s_vis);
-    }
+    tile_item<KVT, D, kPow2Block>(a, item, tid, s_table, s_kv, s_kv + kRows, s_vis);
   }
 }
 
@@ -1523,45 +1672,45 @@ DeviceResources* overlap_for(int device) {
 }
 
 // cus == 0: one workgroup per item (the tile pass alone). cus > 0: a persistent grid beside the
-// row pass, of one workgroup per CU staged straight into LDS (float32 pools beside full-size row
-// workgroups), else of two register-staged workgroups per CU, or of three with
-// PKV_ATTN_DOMINANT_TILES. Measured on MI355X (config 3's shape, 30-240 decode rows):
-//  - float32 beside full rows: one direct-to-LDS workgroup per CU is best while the tile pass's
-//    time is below about 1.1 times the row pass's (1.44 ms against 1.57 / 1.46 ms with two /
-//    three register-staged ones at 120 decode rows), three register-staged ones above it
-//    (0.86 against 0.99 ms at 30 rows);
-//  - bfloat16 (always register-staged): one per CU leaves the tile pass far behind (1.82 ms at
-//    120 decode rows), two are best below the same crossover (1.11 ms), three above it;
-//  - beside lean row workgroups the 100 KiB of direct-to-LDS stages would crowd them out (the
-//    prefix-sharing step's attention took 0.30 instead of 0.23 ms); one, two or three
-//    register-staged workgroups per CU tie there in float32, and two are best in bfloat16
-//    (0.146 against 0.173 ms with one).
+// row pass. Measured on MI355X, 8 chunks of 512 rows beside 30-240 decode rows and the
+// 256-sequence prefix-sharing step:
+//  - float32 beside full-size row workgroups: one per CU is best while the tile pass is the
+//    shorter one (120 rows: 1.58 ms against 1.74 with two), PKV_ATTN_DOMINANT_TILES takes as many
+//    as fit (60 rows 1.08 against 1.26 ms, 30 rows 0.89 against 1.23);
+//  - bfloat16: one, two or three per CU are within 2% at every balance (120 rows 0.875-0.90 ms);
+//  - float32 beside lean row workgroups (prefix sharing): the float32 products, two per CU. The
+//    split tiles' 58 KiB of LDS and 237 VGPRs leave one lean row workgroup on the CU (0.303 ms
+//    the step against 0.271; 0.332 with one per CU, 0.292 with the passes one after the other).
+// PKV_ATTN_DOMINANT_TILES changes the grid only, never the products.
 template <typename KVT, int D>
 int launch_tiles(const Params& a, int64_t num_tiles, int64_t cus, bool lean_rows, hipStream_t stream) {
   if constexpr (D % 16 == 0 && D >= 32) {
     const int64_t items = num_tiles * static_cast<int64_t>(a.max_parts) * a.num_heads;
     if (items > 0x7fffffff) return PKV_EUNSUPPORTED;
     const bool pow2 = (a.block_size & (a.block_size - 1)) == 0;
-    constexpr bool kDmaType = PKV_TILE_DMA && std::is_same_v<KVT, float>;
-    const bool block_fits = static_cast<int64_t>(a.block_size) * a.num_heads * D <= INT32_MAX;
     const bool dominant = (a.flags & PKV_ATTN_DOMINANT_TILES) != 0;
-    const bool dma = kDmaType && cus > 0 && !lean_rows && !dominant && block_fits;
-    const int64_t max_groups = cus * (dma ? 1 : dominant ? 3 : 2);
+    const bool beside = cus > 0;
+    constexpr bool kF32 = std::is_same_v<KVT, float>;
+    const bool split = !(kF32 && beside && lean_rows);
+    const int64_t max_groups = cus * (dominant ? 3 : kF32 && split ? 1 : 2);
     const int64_t groups = max_groups > 0 && max_groups < items ? max_groups : items;
     const dim3 grid(static_cast<uint32_t>(groups));
     const auto n = static_cast<uint32_t>(items);
-    const size_t stage_bytes = kTileStages * TileShape<D>::kStageFloats * sizeof(float);
-    if (dma && pow2) {
-      hipLaunchKernelGGL((tile_partial_kernel<KVT, D, true, kDmaType>), grid, dim3(kTileThreads), stage_bytes,
-                         stream, a, n);
-    } else if (dma) {
-      hipLaunchKernelGGL((tile_partial_kernel<KVT, D, false, kDmaType>), grid, dim3(kTileThreads), stage_bytes,
-                         stream, a, n);
-    } else if (pow2) {
-      hipLaunchKernelGGL((tile_partial_kernel<KVT, D, true, false>), grid, dim3(kTileThreads), 0, stream, a, n);
-    } else {
-      hipLaunchKernelGGL((tile_partial_kernel<KVT, D, false, false>), grid, dim3(kTileThreads), 0, stream, a, n);
+    auto launch = [&](auto path) {
+      constexpr TilePath kPath = decltype(path)::value;
+      if (pow2) {
+        hipLaunchKernelGGL((tile_partial_kernel<KVT, D, true, kPath>), grid, dim3(kTileThreads), 0, stream, a, n);
+      } else {
+        hipLaunchKernelGGL((tile_partial_kernel<KVT, D, false, kPath>), grid, dim3(kTileThreads), 0, stream, a, n);
+      }
+    };
+    if constexpr (kF32) {
+      if (!split) {
+        launch(std::integral_constant<TilePath, TilePath::kFloat>{});
+        return check_launch();
+      }
     }
+    launch(std::integral_constant<TilePath, TilePath::kSplit>{});
     return check_launch();
   } else {
     return PKV_EUNSUPPORTED;

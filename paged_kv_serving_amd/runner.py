@@ -11,7 +11,7 @@ enqueued by one C++ call of the host extension:
     pkv_rope_append     : RoPE on q (in place) and k, and the scatter of the rotated keys and the
                           values into their slots, in one launch
     pkv_paged_attention : every query of the ragged batch against its block table in one call:
-                          decode rows stream K/V per row, prefill runs go to the fp32 MFMA tile
+                          decode rows stream K/V per row, prefill runs go to the MFMA tile
                           pass, then the split-context reduce when a context spans partitions
     rocBLAS sgemm, pkv_silu_mul : the output projection and the SwiGLU block
 

@@ -1175,3 +1175,59 @@ def test_empty_inputs_leave_the_pools_alone(device) -> None:
     assert ops.greedy_tokens(torch.zeros((0, 16), device=device)).shape == (0,)
     torch.cuda.synchronize()
     assert torch.equal(keys, before[0]) and torch.equal(values, before[1])
+
+
+@pytest.mark.parametrize("kv", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim", [32, 64, 128, 256])
+@pytest.mark.parametrize("block", [3, 16])
+def test_tiles_with_infinite_values_fall_back_to_float32_products(device, kv, dim, block) -> None:
+    """A tile's products run on exact bfloat16 pieces, which an infinity does not survive, so a
+    tile that meets one is computed with float32 products: a key of -inf (times a positive query
+    component) takes no weight, an infinite value reaches the rows that see it and no other
+    tile, and every other row stays within the tolerance of the float64 result. Chunks of 17, 64,
+    65 and 130 rows (parts of a wavefront, whole and split tiles) from offset 40."""
+    say("infinite values", kv, dim, block)
+    rng = np.random.default_rng(dim + block)
+    heads, offset = 2, 40
+    for rows in (17, 64, 65, 130):
+        context = offset + rows
+        pool = -(-context // block) + 3
+        kc, vc = (rng.standard_normal((pool, block, heads, dim)).astype(np.float32) for _ in range(2))
+        if kv == "bfloat16":
+            kc, vc = bf16_round(kc), bf16_round(vc)
+        table = rng.permutation(pool)[: -(-context // block)]
+        q = rng.standard_normal((rows, heads, dim)).astype(np.float32)
+        q[:, :, 0] = np.abs(q[:, :, 0]) + 0.5
+        flat = table[np.arange(context) // block] * block + np.arange(context) % block
+        keys, values = kc.reshape(-1, heads, dim), vc.reshape(-1, heads, dim)
+        keys[flat[5], :, 0] = -np.inf
+        values[flat[context - 1], :, 1] = np.inf  # only the last row sees this key
+        positions = np.arange(offset, context)
+        k64, v64 = keys[flat].astype(np.float64), values[flat].astype(np.float64)
+        scores = np.einsum("thd,khd->htk", q.astype(np.float64), k64) * dim**-0.5
+        scores[:, np.arange(context)[None, :] > positions[:, None]] = -np.inf
+        p = np.exp(scores - scores.max(-1, keepdims=True))
+        v64[context - 1, :, 1] = 0.0
+        want = np.einsum("htk,khd->thd", p / p.sum(-1, keepdims=True), v64)
+        args = (
+            torch.from_numpy(q).to(device), torch.from_numpy(positions.astype(np.int32)).to(device),
+            torch.zeros(rows, dtype=torch.int32, device=device),
+            torch.from_numpy(kc).to(device).to(getattr(torch, kv)), torch.from_numpy(vc).to(device).to(getattr(torch, kv)),
+            torch.from_numpy(table.astype(np.int32)[None]).to(device),
+            torch.tensor([context], dtype=torch.int32, device=device), dim**-0.5,
+        )  # fmt: skip
+        seq = np.zeros(rows, np.int64)
+        for end in (0, ops.TILE_WHOLE):
+            _, tiles = ops.plan_rows(seq, dim)
+            tiles[:, 3] = end
+            plan = ops.upload_plan(np.zeros((0, 2), np.int32), tiles, device)
+            got = ops.paged_attention_ragged(*args, max_context_len=context, plan=plan).cpu().numpy()
+            # The wavefronts (16 rows) of the last tile that reach the infinite value's step of 32
+            # keys (16 at head_dim 256) multiply it, by zero or not.
+            step = 16 if dim == 256 else 32
+            first = next(r for r in range((rows - 1) // 64 * 64, rows, 16)
+                         if offset + min(r + 16, rows) > (context - 1) // step * step)  # fmt: skip
+            assert np.isinf(got[-1, :, 1]).all()
+            clean = np.ones(got.shape, bool)
+            clean[first:, :, 1] = False
+            assert np.max(np.abs(np.where(clean, got, 0) - np.where(clean, want, 0))) < FP32_TOL, (rows, end)
