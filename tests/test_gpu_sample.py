@@ -58,3 +58,22 @@ def test_strided_and_misaligned_rows(device) -> None:
     assert np.array_equal(got, _argmax_rows(big[:, 1:258].cpu().numpy()))
     aligned = big[::2, :256]  # stride 600, aligned: the vector path
     assert np.array_equal(ops.greedy_tokens(aligned).cpu().numpy(), _argmax_rows(aligned.cpu().numpy()))
+
+
+@pytest.mark.parametrize("vocab", [1, 2, 3, 5, 4095, 4096, 4099, 16_387, 50_257])
+def test_every_alignment_and_edge_of_a_row(device, vocab) -> None:
+    """Rows start at each of the four offsets from a 16-byte boundary, with the maximum at the
+    row's ends and around its aligned body's ends (the first three and last four ids), at ids a
+    workgroup's stride of 4,096 apart (ties go to the lowest) and with a NaN behind each."""
+    picks = sorted({i % vocab for i in (0, 1, 2, 3, -1, -2, -3, -4, 4095, 4096, 4100, vocab // 2)})
+    for offset in range(4):
+        rows = np.full((2 * len(picks), vocab), -1.0, dtype=np.float32)
+        for r, i in enumerate(picks):
+            rows[r, i:: 4096] = 7.0
+            rows[len(picks) + r, 0] = np.inf
+            rows[len(picks) + r, i:: 4096] = np.nan
+        held = torch.zeros((rows.shape[0], vocab + 4), device=device)
+        flat = held.view(-1)[offset : offset + rows.size].view(rows.shape)  # rows vocab apart
+        flat.copy_(torch.from_numpy(rows))
+        got = ops.greedy_tokens(flat).cpu().numpy()
+        assert np.array_equal(got, _argmax_rows(rows)), (offset, got)
