@@ -10,9 +10,11 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from oracle.model import rms_norm as oracle_rms_norm
 from oracle.model import silu as oracle_silu
+from paged_kv_serving_amd import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -119,3 +121,35 @@ def test_gather_rows_picks_rows_and_zeroes_ids_outside_the_table(device, width, 
         want = src[i, :width] if 0 <= i < 50 else np.zeros(width, np.float32)
         assert np.array_equal(got[r, :width], want), r
         assert np.all(got[r, width:] == 5.0)  # nothing past the row's width is written
+
+
+@pytest.mark.parametrize("dim", [4, 256, 260, 1024, 1028, 4095, 4096, 4100, 16_384, 16_388])
+def test_rms_norm_at_the_edges_of_its_row_layouts(device, dim) -> None:
+    """A wavefront, 256 or 1024 threads per row, and the scalar kernel (16,388 floats, rows off a
+    16-byte boundary), each with and without the residual add, against float64: the sum of squares
+    of n terms in at least 64 partial sums, a quotient and a product stay within 2e-6."""
+    rng = np.random.default_rng(dim)
+    for rows, pad in ((1, 0), (5, 0), (3, 1), (4, 4)):
+        x, d = (rng.standard_normal((rows, dim)).astype(np.float32) for _ in range(2))
+        w = rng.standard_normal(dim).astype(np.float32)
+        for delta in (None, d):
+            held = torch.zeros((rows, dim + pad), device=device)
+            hidden = held[:, pad:]
+            hidden.copy_(torch.from_numpy(x))
+            got = ops.rms_norm(hidden, _to(device, w), 1e-5, delta=None if delta is None else _to(device, d))
+            h = x if delta is None else x + d
+            assert np.array_equal(hidden.cpu().numpy(), h)
+            h64 = h.astype(np.float64)
+            want = h64 / np.sqrt(np.mean(h64**2, axis=1, keepdims=True) + 1e-5) * w
+            np.testing.assert_allclose(got.cpu().numpy(), want, rtol=2e-6, atol=1e-12)
+
+
+@pytest.mark.parametrize(("rows", "width"), [(1, 4), (3, 1020), (2, 1024), (2, 1028), (70_000, 4), (5, 1030)])
+def test_silu_mul_vectors_and_rows_past_the_grid(device, rows, width) -> None:
+    """Whole and partial chunks of 1,024 elements, more rows than the grid's 65,535, and a width
+    that takes the one-element kernel; relative 1e-6 of float64, as the oracle test."""
+    rng = np.random.default_rng(width)
+    gate_up = (4 * rng.standard_normal((rows, 2 * width))).astype(np.float32)
+    got = ops.silu_mul(_to(device, gate_up), width).cpu().numpy()
+    g, u = gate_up[:, :width].astype(np.float64), gate_up[:, width:].astype(np.float64)
+    np.testing.assert_allclose(got, g / (1 + np.exp(-g)) * u, rtol=1e-6, atol=1e-12)
