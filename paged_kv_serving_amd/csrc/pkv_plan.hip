@@ -19,7 +19,17 @@
 //      the rows start the row pass after the prefix.
 //   4. Partition size: the one whose whole partitions (<= 1024 keys) cover the largest group's
 //      prefix with about 512 tile workgroups; without groups 1024 when rows x heads x
-//      ceil(context / 1024) >= 8192, else 512. An explicit size is kept.
+//      ceil(context / 1024) >= 8192, else 512. A call of partitioned tiles alone takes the largest
+//      of 512, 256 and 128 keys that makes 200 (tile, head, partition) items, or 128, if the
+//      split-context workspace stays within PKV_STATIC_SCRATCH_BYTES: a tile walks its keys in one
+//      serial chain, so a few tiles must be split to occupy 256 CUs, while splitting more of them
+//      costs set-up and the reduce (so 128 items are enough where no tile is split: 4 x 200 rows
+//      behind up to 300, 12 x 64 heads, 23.6 us at 512 keys and 24.5 at 256, bfloat16 16.7 and
+//      19.4). Measured at 1024 / 512 / 128 keys: 64 rows behind 1000, 8 x 128
+//      heads, float32 68.8 / 40.6 / 20.0 us, bfloat16 42.4 / 27.4 / 16.4; 301 behind 1500, 32 x
+//      128, 86.8 / 75.7 / 90.9 and 49.8 / 41.4 / 62.3; 3 x 150 behind up to 200, 32 x 128, 31.1 /
+//      31.1 / 36.8 and 20.4 / 20.4 / 27.6; 301 behind 150, 16 x 64, 21.7 / 21.7 / 18.9 and 16.2 /
+//      16.2 / 16.4. An explicit size is kept.
 //   5. PKV_ATTN_SHARED_KV when >= 25% of the block ids the row pass still reads repeat;
 //      PKV_ATTN_SHORT_ROWS when the row-pass items average < 256 keys; PKV_ATTN_DOMINANT_TILES
 //      when the call has both passes and the tile pass's estimated time is at least 1.1 times
@@ -52,6 +62,8 @@ constexpr int64_t kShortRowKeys = 256;
 constexpr int64_t kDominantTileWeight = 34;  // rule 5: tile_keys * 34 >= row_keys * esize * 275
 constexpr int64_t kDominantRowWeight = 275;
 constexpr int kDefaultPlanPartition = 512;
+constexpr int64_t kTargetTileItems = 200;  // rule 4: a workgroup on most of 256 CUs
+constexpr int64_t kTargetUnsplitItems = 128;
 
 struct Tile {
   int32_t first, count, begin, end;
@@ -225,6 +237,27 @@ int64_t distinct_count(std::vector<int32_t>& ids) {
   return std::unique(ids.begin(), ids.end()) - ids.begin();
 }
 
+// Rule 4 for a call of partitioned tiles alone; `otherwise` when its workspace would not fit the
+// library's static scratch.
+int32_t tile_partition(const std::vector<Tile>& tiles, const std::vector<int64_t>& vis, int32_t num_heads,
+                       int32_t head_dim, int64_t max_context, int32_t otherwise) {
+  std::vector<int64_t> longest;
+  longest.reserve(tiles.size());
+  for (const Tile& t : tiles) {
+    longest.push_back(*std::max_element(vis.begin() + t.first, vis.begin() + t.first + t.count));
+  }
+  const int64_t longest_of_all = *std::max_element(longest.begin(), longest.end());
+  int32_t size = 512;
+  for (; size > 128; size /= 2) {
+    int64_t items = 0;
+    for (const int64_t v : longest) items += std::max<int64_t>(1, ceil_div(v, size)) * num_heads;
+    if (items >= (longest_of_all > size ? kTargetTileItems : kTargetUnsplitItems)) break;
+  }
+  const int64_t parts = ceil_div(max_context, size);  // as pkv_attention_workspace_bytes counts them
+  const int64_t bytes = static_cast<int64_t>(vis.size()) * num_heads * parts * (head_dim + 2) * 4;
+  return bytes <= PKV_STATIC_SCRATCH_BYTES ? size : otherwise;
+}
+
 int32_t prefix_partition(int64_t shared_tokens, int64_t tiles, int32_t num_heads) {
   int32_t best = 0;
   for (int64_t k = std::max<int64_t>(1, ceil_div(shared_tokens, 1024));; ++k) {
@@ -343,14 +376,18 @@ extern "C" int pkv_plan_batch(const int32_t* query_seq, const int32_t* query_pos
       partition = prefix_partition(largest->common * block_size, tile_count, num_heads);
     }
     if (partition == 0) {
-      int64_t n_present = 0, wide = 0;
+      int64_t n_present = 0, wide = 0, max_context = 0;
       for (int32_t s = 0; s < num_seqs; ++s) {
         if (!present[s]) continue;
         ++n_present;
         wide += ceil_div(context_lens[s], 1024);
+        max_context = std::max<int64_t>(max_context, context_lens[s]);
       }
       const int64_t per_seq = std::max<int64_t>(1, num_queries / n_present);
       partition = wide * per_seq * num_heads >= kWidePartitionItems ? 1024 : 512;
+      if (row_pass.empty() && tiles[0].end != PKV_TILE_WHOLE) {
+        partition = tile_partition(tiles, vis, num_heads, head_dim, max_context, partition);
+      }
     }
   }
 

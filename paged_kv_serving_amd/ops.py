@@ -423,6 +423,10 @@ MIN_PREFIX_PARTITION = 256
 #: final rows written directly, nothing for the reduce) once the call has at least this many
 #: (tile, head) workgroups: four per CU of 256 keeps the chip full without splitting contexts.
 WHOLE_TILE_GROUPS = 1024
+#: (tile, head, partition) items the partition choice of a call of partitioned tiles alone aims for.
+TARGET_TILE_ITEMS = 200
+#: ... and the items that are enough where no tile spans two partitions (no reduce follows).
+TARGET_UNSPLIT_ITEMS = 128
 #: Tile record end partition of a whole tile (include/pkv.h PKV_TILE_WHOLE).
 TILE_WHOLE = -1
 #: Row-pass items shorter than this many keys on average launch the lighter row-pass workgroup
@@ -578,6 +582,25 @@ def _prefix_partition(shared_tokens: int, tiles: int, num_heads: int) -> int:
             break
         k += 1
     return best
+
+
+def _tile_partition(
+    tiles: np.ndarray, visible: np.ndarray, num_heads: int, head_dim: int, max_context: int, otherwise: int
+) -> int:  # fmt: skip
+    """Partition size of a call of partitioned tiles alone: the largest of 512, 256 and 128 keys
+    that makes TARGET_TILE_ITEMS (tile, head, partition) items, or TARGET_UNSPLIT_ITEMS where it
+    splits no tile (and no reduce follows), or 128; ``otherwise`` when the
+    split-context workspace would not fit the library's static scratch. A tile walks its keys in
+    one serial chain, so a few tiles have to be split to fill the GPU."""
+    longest = np.fromiter((visible[f : f + c].max() for f, c in tiles[:, :2].tolist()), np.int64, tiles.shape[0])
+    size = 512
+    while size > 128:
+        items = int(np.maximum(1, -(-longest // size)).sum()) * num_heads
+        if items >= (TARGET_TILE_ITEMS if longest.max() > size else TARGET_UNSPLIT_ITEMS):
+            break
+        size //= 2
+    need = visible.size * num_heads * -(-max_context // size) * (head_dim + 2) * 4
+    return size if need <= _native.STATIC_SCRATCH_BYTES else otherwise
 
 
 def _visible(seq: np.ndarray, contexts: np.ndarray, positions: np.ndarray | None) -> np.ndarray:
@@ -736,6 +759,8 @@ def plan_batch(
             partition = _prefix_partition(largest[2] * block_size, tile_count, num_heads)
         if partition == 0:
             partition = _wide_partition(contexts[present], num_heads, max(1, seq.size // present.size))
+            if rows.size == 0 and tiles[0, 3] != TILE_WHOLE:
+                partition = _tile_partition(tiles, visible, num_heads, head_dim, int(contexts[present].max()), partition)
     prefix_tiles = []
     for start, count, common in groups:
         parts = common * block_size // partition
