@@ -415,6 +415,20 @@ int pkv_gather_rows(float* out, int64_t out_stride, const float* src, int64_t sr
                     int device, void* stream);
 
 /*
+ * The int32 metadata of an attention call over one sequence, in one buffer:
+ *     out = [positions (num_queries) | num_queries zeros | block_table (num_blocks) | context_len]
+ * i.e. the query positions, every query's sequence index, the one-row table and its context length.
+ *
+ * No counterpart in the reference, whose attention takes one sequence at a time
+ * (src/paged_kv_serving/engine/attention.py:42-50). positions and block_table are device integers
+ * of position_bytes / table_bytes each (4 or 8), narrowed to 32 bits; out holds 2 * num_queries +
+ * num_blocks + 1 values.
+ */
+int pkv_sequence_metadata(int32_t* out, const void* positions, int32_t position_bytes,
+                          int64_t num_queries, const void* block_table, int32_t table_bytes,
+                          int64_t num_blocks, int32_t context_len, int device, void* stream);
+
+/*
  * Greedy sampling: the argmax of each logits row, on the device.
  *
  * Replaces src/paged_kv_serving/engine/sampling.py:28-30 (greedy_token: int(np.argmax(logits)))

@@ -90,6 +90,7 @@ EXPORTED_SYMBOLS = (
     "pkv_rms_norm",
     "pkv_silu_mul",
     "pkv_gather_rows",
+    "pkv_sequence_metadata",
 )
 
 
@@ -316,6 +317,10 @@ def _declare(lib: ctypes.CDLL) -> None:
         _ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _i32, _c_int, _ptr,  # out, stride, src, stride, src rows, index, rows, width, device, stream
     ]
     lib.pkv_gather_rows.restype = _c_int
+    lib.pkv_sequence_metadata.argtypes = [
+        _ptr, _ptr, _i32, _i64, _ptr, _i32, _i64, _i32, _c_int, _ptr,  # out, positions, bytes, queries, table, bytes, blocks, context, device, stream
+    ]
+    lib.pkv_sequence_metadata.restype = _c_int
 
 
 def library() -> ctypes.CDLL:

@@ -15,7 +15,7 @@ import threading
 import numpy as np
 import torch
 
-from paged_kv_serving_amd import ops
+from paged_kv_serving_amd import _native, ops
 
 __all__ = ["DEFAULT_TILE_BLOCKS", "paged_attention"]
 
@@ -55,6 +55,12 @@ def _to_device(value, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
     if isinstance(value, torch.Tensor):
         return value.to(device=device, dtype=dtype)
     return torch.as_tensor(np.asarray(value), dtype=dtype).to(device)
+
+
+def _is_index_vector(value, device: torch.device) -> bool:
+    """Whether ``value`` is a contiguous 1-D int32 or int64 tensor on the HIP device ``device``."""
+    return (isinstance(value, torch.Tensor) and value.dtype in (torch.int64, torch.int32) and value.dim() == 1
+            and value.device == device and device.type == "cuda" and value.is_contiguous())  # fmt: skip
 
 
 def paged_attention(
@@ -105,11 +111,23 @@ def paged_attention(
     keys, values = keys.contiguous(), values.contiguous()
     q = _to_device(queries, torch.float32, device).contiguous()
     num_queries = q.shape[0]
-    positions = _to_device(query_positions, torch.int32, device)
-    query_seq = torch.zeros(num_queries, dtype=torch.int32, device=device)
     used = -(-context_len // block_size)
-    table = _to_device(block_table, torch.int32, device)[:used].reshape(1, used).contiguous()
-    context = torch.full((1,), int(context_len), dtype=torch.int32, device=device)  # no host copy
+    if _is_index_vector(query_positions, device) and _is_index_vector(block_table, device) and context_len < 1 << 31:
+        # All the integer metadata in one buffer, by one launch.
+        meta = torch.empty(2 * num_queries + used + 1, dtype=torch.int32, device=device)
+        index = device.index
+        rc = _native.library().pkv_sequence_metadata(
+            meta.data_ptr(), query_positions.data_ptr(), query_positions.element_size(), num_queries,
+            block_table.data_ptr(), block_table.element_size(), used, int(context_len), index, ops._stream(index),
+        )  # fmt: skip
+        _native.check(rc, "pkv_sequence_metadata")
+        positions, query_seq, table, context = meta.split((num_queries, num_queries, used, 1))
+        table = table.view(1, used)
+    else:
+        positions = _to_device(query_positions, torch.int32, device)
+        query_seq = torch.zeros(num_queries, dtype=torch.int32, device=device)
+        table = _to_device(block_table, torch.int32, device)[:used].reshape(1, used).contiguous()
+        context = torch.full((1,), int(context_len), dtype=torch.int32, device=device)  # no host copy
     out = ops.paged_attention_ragged(
         q, positions, query_seq, keys, values, table, context, scale,
         max_context_len=int(context_len),

@@ -192,8 +192,58 @@ __global__ __launch_bounds__(kNormThreads) void gather_rows_kernel(float* __rest
   }
 }
 
+// The int32 metadata of a call over one sequence: out = positions, one zero per query (its sequence
+// index), the table and the context length. One launch of a few hundred bytes in place of four
+// framework kernels (two casts, two fills): the 1 x 256-key call 36.5 -> 23.7 us, which the host's
+// launches bound.
+template <typename PositionT, typename BlockT>
+__global__ __launch_bounds__(kNormThreads) void sequence_metadata_kernel(int32_t* __restrict__ out,
+                                                                         const PositionT* __restrict__ positions,
+                                                                         int64_t num_queries,
+                                                                         const BlockT* __restrict__ table,
+                                                                         int64_t num_blocks, int32_t context_len) {
+  const int64_t total = 2 * num_queries + num_blocks + 1;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x; i < total;
+       i += static_cast<int64_t>(gridDim.x) * kNormThreads) {
+    int32_t v = 0;
+    if (i < num_queries) {
+      v = static_cast<int32_t>(positions[i]);
+    } else if (i >= 2 * num_queries) {
+      const int64_t b = i - 2 * num_queries;
+      v = b < num_blocks ? static_cast<int32_t>(table[b]) : context_len;
+    }
+    out[i] = v;
+  }
+}
+
 }  // namespace
 }  // namespace pkv
+
+extern "C" int pkv_sequence_metadata(int32_t* out, const void* positions, int32_t position_bytes,
+                                     int64_t num_queries, const void* block_table, int32_t table_bytes,
+                                     int64_t num_blocks, int32_t context_len, int device, void* stream) {
+  using namespace pkv;
+  if (num_queries < 0 || num_blocks < 0 || (position_bytes != 4 && position_bytes != 8) ||
+      (table_bytes != 4 && table_bytes != 8) || !out || (num_queries > 0 && !positions) ||
+      (num_blocks > 0 && !block_table)) {
+    return PKV_EINVAL;
+  }
+  DeviceGuard guard(device);
+  if (!guard.ok()) return PKV_EHIP;
+  (void)hipGetLastError();
+  const int64_t wanted = (2 * num_queries + num_blocks + 1 + kNormThreads - 1) / kNormThreads;
+  const dim3 grid(static_cast<uint32_t>(wanted < 1024 ? wanted : 1024));
+  auto launch = [&](auto position, auto block) {
+    using P = decltype(position);
+    using B = decltype(block);
+    hipLaunchKernelGGL((sequence_metadata_kernel<P, B>), grid, dim3(kNormThreads), 0,
+                       static_cast<hipStream_t>(stream), out, static_cast<const P*>(positions), num_queries,
+                       static_cast<const B*>(block_table), num_blocks, context_len);
+    return check_launch();
+  };
+  if (position_bytes == 8) return table_bytes == 8 ? launch(int64_t{}, int64_t{}) : launch(int64_t{}, int32_t{});
+  return table_bytes == 8 ? launch(int32_t{}, int64_t{}) : launch(int32_t{}, int32_t{});
+}
 
 extern "C" int pkv_gather_rows(float* out, int64_t out_stride, const float* src, int64_t src_stride,
                                int64_t src_rows, const int64_t* index, int64_t num_rows, int32_t width,

@@ -154,3 +154,32 @@ def test_host_calls_of_changing_sizes_reuse_the_staging_buffer(device) -> None:
         want = dense_attention(q, gather_context(kc, table, length), gather_context(vc, table, length), scale, pos)
         got = paged_attention(q, pos, kc, vc, table, length, scale)
         assert np.max(np.abs(got - want)) < TOL, (length, heads, dim)
+
+
+@pytest.mark.parametrize("queries", [1, 3, 300])
+@pytest.mark.parametrize("where", ["int64", "int32", "mixed", "strided", "float", "cpu"])
+def test_every_form_of_positions_and_table_gives_the_same_rows(device, queries, where) -> None:
+    """Positions and table as contiguous int32 or int64 device vectors (narrowed by one launch with
+    the rest of the metadata) and in the forms that take the general conversion: strided views,
+    float positions, host tensors. A table longer than the context needs is read up to it."""
+    length = 301
+    blocks = -(-length // BLOCK) + 5
+    keys, values, flat_k, flat_v = build_cache(length, blocks)
+    q = np.random.default_rng(queries).standard_normal((queries, HEADS, DIM)).astype(np.float32)
+    pos = np.arange(length - queries, length)
+    want = dense_attention(q, flat_k, flat_v, DIM**-0.5, pos)
+    positions, table = torch.from_numpy(pos), torch.arange(blocks)
+    if where in ("int32", "mixed"):
+        positions = positions.to(torch.int32)
+    if where == "int32":
+        table = table.to(torch.int32)
+    if where == "float":
+        positions = positions.double()
+    if where != "cpu":
+        positions, table = positions.to(device), table.to(device)
+    if where == "strided":
+        positions = torch.stack([positions, positions], dim=1)[:, 0]
+        table = torch.stack([table, table], dim=1)[:, 0]
+    to = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    out = paged_attention(to(q), positions, to(keys), to(values), table, length, DIM**-0.5)
+    assert out.is_cuda and np.max(np.abs(out.cpu().numpy() - want)) < TOL
