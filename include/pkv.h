@@ -429,6 +429,66 @@ int pkv_sequence_metadata(int32_t* out, const void* positions, int32_t position_
                           int64_t num_blocks, int32_t context_len, int device, void* stream);
 
 /*
+ * A float32 matrix product of a small decoder with the row-wise steps around it, in one launch:
+ *     x   = input rows (of a row_index: PKV_LINEAR_LOGITS), RMS-normalised except PKV_LINEAR_ADD
+ *     y   = x @ weights
+ *     PKV_LINEAR_ADD         : output += y                       (out_proj, down_proj + residual)
+ *     PKV_LINEAR_SWIGLU      : output = silu(y[:, :cols]) * y[:, cols:]     (weights [gate | up])
+ *     PKV_LINEAR_ROPE_APPEND : y = q | k | v; output = rope(q), the pools' rows at the slots =
+ *                              rope(k) and v
+ *     PKV_LINEAR_LOGITS      : output = y, weights given transposed (the tied embedding)
+ *
+ * Replaces src/paged_kv_serving/engine/model.py:43-46 (rms_norm), :49-51 (silu), :70-81 and
+ * :248-252 (QKV, apply_rope), :256-264 and :283 (the feed-forward block, the residual adds and the
+ * logits) and runner.py:195-196, 215-227, as pkv_rms_norm, a library product, and pkv_rope_append,
+ * pkv_silu_mul, or pkv_gather_rows do, with the same float32 operations in another summation order.
+ *
+ *   input        : row r at r * input_stride, `depth` floats, 16-byte aligned rows.
+ *   weights      : [depth, cols] ([depth, 2 * cols] for SWIGLU) at weight_stride per depth row;
+ *                  LOGITS: [cols, depth] at weight_stride per column, 16-byte aligned.
+ *   norm_weight  : [depth], 16-byte aligned.
+ *   output       : row r at r * output_stride. It must not overlap the input.
+ * depth must be a multiple of 16 and at most PKV_LINEAR_MAX_DEPTH, head_dim 32 or 64 for
+ * ROPE_APPEND. A row index outside [0, input_rows) is a row of zeros; positions and slots are
+ * checked as pkv_rope_append checks them.
+ */
+#define PKV_LINEAR_ADD 0
+#define PKV_LINEAR_SWIGLU 1
+#define PKV_LINEAR_ROPE_APPEND 2
+#define PKV_LINEAR_LOGITS 3
+#define PKV_LINEAR_MAX_DEPTH 1536
+
+typedef struct pkv_linear {
+  const float* input;
+  const float* weights;
+  const float* norm_weight;
+  float* output;
+  int64_t input_stride;
+  int64_t weight_stride;
+  int64_t output_stride;
+  int64_t rows;
+  int32_t kind; /* PKV_LINEAR_* */
+  int32_t cols;
+  int32_t depth;
+  float eps;
+  const int64_t* row_index; /* LOGITS: the input row of each output row */
+  int64_t input_rows;
+  const int64_t* positions; /* ROPE_APPEND, as pkv_rope_append's */
+  const int64_t* slots;
+  const float* cos_table;
+  const float* sin_table;
+  int64_t table_rows;
+  void* key_pool;
+  void* value_pool;
+  int64_t num_slots;
+  int32_t num_heads;
+  int32_t head_dim;
+  int32_t pool_dtype;
+} pkv_linear;
+
+int pkv_linear_forward(const pkv_linear* args, int device, void* stream);
+
+/*
  * Greedy sampling: the argmax of each logits row, on the device.
  *
  * Replaces src/paged_kv_serving/engine/sampling.py:28-30 (greedy_token: int(np.argmax(logits)))

@@ -38,7 +38,7 @@ INCLUDE = REPO_ROOT / "include"
 LIB_PATH = PACKAGE_DIR / "libpkv.so"
 SOURCES = (
     CSRC / "pkv_copy.hip", CSRC / "pkv_rope.hip", CSRC / "pkv_attention.hip", CSRC / "pkv_sample.hip",
-    CSRC / "pkv_plan.hip", CSRC / "pkv_model.hip",
+    CSRC / "pkv_plan.hip", CSRC / "pkv_model.hip", CSRC / "pkv_linear.hip",
 )
 
 # gfx950 only. Packed-FP32 VALU instructions are disabled: the code relies on scalar fp32 FMA.
@@ -91,6 +91,7 @@ EXPORTED_SYMBOLS = (
     "pkv_silu_mul",
     "pkv_gather_rows",
     "pkv_sequence_metadata",
+    "pkv_linear_forward",
 )
 
 
@@ -202,7 +203,7 @@ def bound_host():
                          address(lib.hipGetDevice), address(lib.hipSetDevice),
                          address(lib.hipEventCreateWithFlags), address(lib.hipEventRecord),
                          address(lib.hipEventSynchronize), address(lib.hipEventDestroy),
-                         address(lib.pkv_append))  # fmt: skip
+                         address(lib.pkv_append), address(lib.pkv_linear_forward))  # fmt: skip
                 _BOUND = True
     return ext
 
@@ -321,6 +322,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         _ptr, _ptr, _i32, _i64, _ptr, _i32, _i64, _i32, _c_int, _ptr,  # out, positions, bytes, queries, table, bytes, blocks, context, device, stream
     ]
     lib.pkv_sequence_metadata.restype = _c_int
+    lib.pkv_linear_forward.argtypes = [_ptr, _c_int, _ptr]  # args, device, stream
+    lib.pkv_linear_forward.restype = _c_int
 
 
 def library() -> ctypes.CDLL:

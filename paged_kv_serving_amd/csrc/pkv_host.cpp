@@ -58,7 +58,7 @@
 //       tens of thousands of blocks); it is left all zero.
 //   bind(plan_batch, paged_attention, paged_attention_append, copy_blocks, rms_norm, silu_mul,
 //        rope_append, memcpy_async[, gather_rows, greedy_tokens, get_device, set_device,
-//        event_create, event_record, event_synchronize, event_destroy, append])
+//        event_create, event_record, event_synchronize, event_destroy, append, linear_forward])
 //       Takes the addresses of those libpkv.so entry points (include/pkv.h), so the calls below
 //       reach the library without ctypes' per-argument conversions, and of hipMemcpyAsync,
 //       hipGetDevice, hipSetDevice and hipEventCreateWithFlags / Record / Synchronize / Destroy
@@ -73,7 +73,9 @@
 //       into the next norm, the [gate | up] product, the SwiGLU gate and the down product; then
 //       the logits rows, their product with the tied embedding, and greedy sampling when an
 //       output address is given. The products are rocBLAS sgemm calls (the rocBLAS the process
-//       has loaded, one handle per device, used by one forward pass at a time). `fields` holds
+//       has loaded, one handle per device, used by one forward pass at a time); a small decoder's
+//       (kSmallRows, kSmallModel) are pkv_linear_forward calls, which take the norms, RoPE + append,
+//       gate, residual adds and row lookup of the logits into the same launches. `fields` holds
 //       the integers of the Field enum below (addresses, sizes, the attention plan); `layers`
 //       one tuple of six weight addresses per layer (attn_norm, qkv, out_proj, ffn_norm,
 //       [gate | up], down). Raises RuntimeError naming the first step that failed.
@@ -834,6 +836,7 @@ decltype(&pkv_silu_mul) g_silu_mul = nullptr;
 decltype(&pkv_rope_append) g_rope_append = nullptr;
 decltype(&pkv_append) g_append = nullptr;
 decltype(&pkv_gather_rows) g_gather_rows = nullptr;
+decltype(&pkv_linear_forward) g_linear = nullptr;  // optional: null takes the library products
 decltype(&pkv_greedy_tokens) g_greedy_tokens = nullptr;
 // hipGetDevice / hipSetDevice of the same runtime, by their C signatures.
 using GetDeviceFn = int (*)(int* device);
@@ -890,10 +893,10 @@ T* ptr(unsigned long long address) {
 PyObject* bind(PyObject*, PyObject* args) {
   unsigned long long plan, attention, attention_append, copy, norm, gate, rope, memcpy_async;
   unsigned long long gather_rows = 0, greedy = 0, get_device = 0, set_device = 0;
-  unsigned long long event_create = 0, event_record = 0, event_synchronize = 0, event_destroy = 0, append = 0;
-  if (!PyArg_ParseTuple(args, "KKKKKKKK|KKKKKKKKK", &plan, &attention, &attention_append, &copy, &norm, &gate, &rope,
+  unsigned long long event_create = 0, event_record = 0, event_synchronize = 0, event_destroy = 0, append = 0, linear = 0;
+  if (!PyArg_ParseTuple(args, "KKKKKKKK|KKKKKKKKKK", &plan, &attention, &attention_append, &copy, &norm, &gate, &rope,
                         &memcpy_async, &gather_rows, &greedy, &get_device, &set_device, &event_create,
-                        &event_record, &event_synchronize, &event_destroy, &append)) {
+                        &event_record, &event_synchronize, &event_destroy, &append, &linear)) {
     return nullptr;
   }
   if (plan == 0 || attention == 0 || attention_append == 0 || copy == 0 || norm == 0 || gate == 0 || rope == 0 ||
@@ -919,6 +922,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   g_event_synchronize = reinterpret_cast<EventFn>(static_cast<uintptr_t>(event_synchronize));
   g_event_destroy = reinterpret_cast<EventFn>(static_cast<uintptr_t>(event_destroy));
   g_append = reinterpret_cast<decltype(g_append)>(static_cast<uintptr_t>(append));
+  g_linear = reinterpret_cast<decltype(g_linear)>(static_cast<uintptr_t>(linear));
   Py_RETURN_NONE;
 }
 
@@ -1462,6 +1466,14 @@ int gemm(void* handle, int64_t m, int64_t n, int64_t k, const float* a, int64_t 
                       static_cast<int32_t>(lda), &zero, c, static_cast<int32_t>(ldc));
 }
 
+// Up to these sizes forward() takes pkv_linear_forward's products (7 launches a layer instead of
+// 10). Measured on MI355X, execute() with its logits back on the host, library products against
+// these: d_model 128 (4 layers, 128 rows) 280 / 205 us, 2 layers of 2 rows 146 / 87, 4 layers of
+// 512 rows 327 / 270; d_model 256 (4 layers) 80 rows 280 / 250, 288 rows 348 / 320, 432 rows 336 /
+// 309; d_model 512 16 rows 245 / 261, 288 rows 413 / 482: there the library's larger tiles win.
+constexpr int64_t kSmallRows = 512;
+constexpr int64_t kSmallModel = 256;
+
 // Integer fields of forward()'s first argument, in order.
 enum Field {
   kDevice, kStream, kTokens, kWanted, kModel, kHeads, kHeadDim, kFf, kVocab,
@@ -1566,21 +1578,62 @@ PyObject* forward(PyObject*, PyObject* args) {
                         static_cast<int32_t>(d), device, stream),
           "pkv_gather_rows (embedding)");
   }
-  if (failed == nullptr) norm(num_layers > 0 ? layer[0] : v[kFinalNorm], nullptr);
+  // A small decoder's products carry the row-wise steps around them in the same launch.
+  const bool small = g_linear != nullptr && num_layers > 0 && T <= kSmallRows && d <= kSmallModel && d % 16 == 0 &&
+                     ff % 16 == 0 && ff <= PKV_LINEAR_MAX_DEPTH && (dim == 32 || dim == 64);
+  if (failed == nullptr && !small) norm(num_layers > 0 ? layer[0] : v[kFinalNorm], nullptr);
+  auto linear = [&](int kind, const float* input, int64_t input_stride, int64_t rows, int64_t depth, int64_t weights,
+                    int64_t weight_stride, int64_t cols, int64_t norm_weight, float* output, int64_t output_stride,
+                    char* kp, char* vp, const char* what) {
+    pkv_linear p{};
+    p.kind = kind;
+    p.input = input;
+    p.input_stride = input_stride;
+    p.rows = rows;
+    p.depth = static_cast<int32_t>(depth);
+    p.weights = ptr<const float>(weights);
+    p.weight_stride = weight_stride;
+    p.cols = static_cast<int32_t>(cols);
+    p.norm_weight = ptr<const float>(norm_weight);
+    p.eps = eps;
+    p.output = output;
+    p.output_stride = output_stride;
+    p.row_index = ptr<const int64_t>(v[kLogitsRows]);
+    p.input_rows = T;
+    p.positions = ptr<const int64_t>(v[kRopePositions]);
+    p.slots = ptr<const int64_t>(v[kSlots]);
+    p.cos_table = ptr<const float>(v[kCos]);
+    p.sin_table = ptr<const float>(v[kSin]);
+    p.table_rows = v[kTableRows];
+    p.key_pool = kp;
+    p.value_pool = vp;
+    p.num_slots = v[kNumSlots];
+    p.num_heads = heads;
+    p.head_dim = dim;
+    p.pool_dtype = static_cast<int32_t>(v[kKvDtype]);
+    return check(g_linear(&p, device, stream), what);
+  };
   const int64_t row = d;  // heads * head_dim
   for (Py_ssize_t l = 0; l < num_layers && failed == nullptr; ++l) {
     const int64_t* w = &layer[6 * l];  // attn_norm, qkv, out_proj, ffn_norm, gate_up, down
     char* kp = ptr<char>(v[kKeyPool]) + l * v[kLayerBytes];
     char* vp = ptr<char>(v[kValuePool]) + l * v[kLayerBytes];
-    // fused = normed @ qkv: [T, 3d], q | k | v per token (model.py:248-249)
-    if (!check(gemm(handle, T, 3 * d, d, normed, d, ptr<const float>(w[1]), 3 * d, false, fused, 3 * d), "rocblas_sgemm (qkv)")) break;
-    // RoPE on q (in place) and k, and the append of k and v (model.py:251-252, runner.py:195-196)
-    if (!check(g_rope_append(fused, 3 * row, fused, fused + row, fused + 2 * row, 3 * row, 3 * row, 3 * row,
-                             ptr<const int64_t>(v[kRopePositions]), ptr<const float>(v[kCos]), ptr<const float>(v[kSin]),
-                             v[kTableRows], kp, vp, static_cast<pkv_dtype>(v[kKvDtype]), v[kNumSlots],
-                             ptr<const int64_t>(v[kSlots]), T, heads, dim, device, stream),
-               "pkv_rope_append")) {
-      break;
+    if (small) {
+      if (!linear(PKV_LINEAR_ROPE_APPEND, hidden, d, T, d, w[1], 3 * d, 3 * d, w[0], fused, 3 * row, kp, vp,
+                  "pkv_linear_forward (qkv)")) {
+        break;
+      }
+    } else {
+      // fused = normed @ qkv: [T, 3d], q | k | v per token (model.py:248-249)
+      if (!check(gemm(handle, T, 3 * d, d, normed, d, ptr<const float>(w[1]), 3 * d, false, fused, 3 * d), "rocblas_sgemm (qkv)")) break;
+      // RoPE on q (in place) and k, and the append of k and v (model.py:251-252, runner.py:195-196)
+      if (!check(g_rope_append(fused, 3 * row, fused, fused + row, fused + 2 * row, 3 * row, 3 * row, 3 * row,
+                               ptr<const int64_t>(v[kRopePositions]), ptr<const float>(v[kCos]), ptr<const float>(v[kSin]),
+                               v[kTableRows], kp, vp, static_cast<pkv_dtype>(v[kKvDtype]), v[kNumSlots],
+                               ptr<const int64_t>(v[kSlots]), T, heads, dim, device, stream),
+                 "pkv_rope_append")) {
+        break;
+      }
     }
     // attention over the pools (runner.py:198-212)
     if (v[kNumPlanRows] > 0 || v[kNumTiles] > 0) {
@@ -1598,6 +1651,17 @@ PyObject* forward(PyObject*, PyObject* args) {
         break;
       }
     }
+    if (small) {
+      if (!linear(PKV_LINEAR_ADD, attended, d, T, d, w[2], d, d, 0, hidden, d, nullptr, nullptr,
+                  "pkv_linear_forward (out_proj)") ||
+          !linear(PKV_LINEAR_SWIGLU, hidden, d, T, d, w[4], 2 * ff, ff, w[3], gated, ff, nullptr, nullptr,
+                  "pkv_linear_forward (gate_up)") ||
+          !linear(PKV_LINEAR_ADD, gated, ff, T, ff, w[5], d, d, 0, hidden, d, nullptr, nullptr,
+                  "pkv_linear_forward (down)")) {
+        break;
+      }
+      continue;
+    }
     // hidden += attended @ out_proj, then the feed-forward norm (model.py:283, 256)
     if (!check(gemm(handle, T, d, d, attended, d, ptr<const float>(w[2]), d, false, tmp, d), "rocblas_sgemm (out_proj)")) break;
     if (!norm(w[3], tmp)) break;
@@ -1613,12 +1677,15 @@ PyObject* forward(PyObject*, PyObject* args) {
   if (failed == nullptr && W > 0) {
     float* picked = f(kPicked);
     float* logits = f(kLogits);
-    if (check(g_gather_rows(picked, d, normed, d, T, ptr<const int64_t>(v[kLogitsRows]), W, static_cast<int32_t>(d),
-                            device, stream),
-              "pkv_gather_rows (logits rows)") &&
-        check(gemm(handle, W, vocab, d, picked, d, ptr<const float>(v[kEmbedding]), d, true, logits, vocab),
-              "rocblas_sgemm (logits)") &&
-        v[kGreedyOut] != 0) {
+    const bool ready = small ? linear(PKV_LINEAR_LOGITS, hidden, d, W, d, v[kEmbedding], d, vocab, v[kFinalNorm], logits,
+                                      vocab, nullptr, nullptr, "pkv_linear_forward (logits)")
+                             : check(g_gather_rows(picked, d, normed, d, T, ptr<const int64_t>(v[kLogitsRows]), W,
+                                                   static_cast<int32_t>(d), device, stream),
+                                     "pkv_gather_rows (logits rows)") &&
+                                   check(gemm(handle, W, vocab, d, picked, d, ptr<const float>(v[kEmbedding]), d, true,
+                                              logits, vocab),
+                                         "rocblas_sgemm (logits)");
+    if (ready && v[kGreedyOut] != 0) {
       check(g_greedy_tokens(ptr<int32_t>(v[kGreedyOut]), logits, vocab, W, vocab, device, stream), "pkv_greedy_tokens");
     }
   }
