@@ -347,7 +347,9 @@ int pkv_paged_attention_append(
  *   context_lens               : int32 [num_seqs], host.
  *   kv_dtype                   : the pools' element type; it weighs the row pass's bytes
  *                                against the tile pass's products for PKV_ATTN_DOMINANT_TILES.
- *   partition_size             : 0 lets the planner choose; a positive value is kept.
+ *   partition_size             : 0 lets the planner choose (for calls of tiles alone, within the
+ *                                static scratch at the longest present context: pass that as
+ *                                max_context_len); a positive value is kept.
  *   min_tile_rows              : the shortest run of one sequence's rows made into tiles (8).
  *   rows_out [rows_capacity, 2], tiles_out [tiles_capacity, 4], merge_out [merge_capacity] :
  *                                int32 outputs in pkv_paged_attention's layout.

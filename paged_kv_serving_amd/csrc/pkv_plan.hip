@@ -19,17 +19,19 @@
 //      the rows start the row pass after the prefix.
 //   4. Partition size: the one whose whole partitions (<= 1024 keys) cover the largest group's
 //      prefix with about 512 tile workgroups; without groups 1024 when rows x heads x
-//      ceil(context / 1024) >= 8192, else 512. A call of partitioned tiles alone takes the largest
-//      of 512, 256 and 128 keys that makes 200 (tile, head, partition) items, or 128, if the
-//      split-context workspace stays within PKV_STATIC_SCRATCH_BYTES: a tile walks its keys in one
-//      serial chain, so a few tiles must be split to occupy 256 CUs, while splitting more of them
-//      costs set-up and the reduce (so 128 items are enough where no tile is split: 4 x 200 rows
-//      behind up to 300, 12 x 64 heads, 23.6 us at 512 keys and 24.5 at 256, bfloat16 16.7 and
-//      19.4). Measured at 1024 / 512 / 128 keys: 64 rows behind 1000, 8 x 128
-//      heads, float32 68.8 / 40.6 / 20.0 us, bfloat16 42.4 / 27.4 / 16.4; 301 behind 1500, 32 x
-//      128, 86.8 / 75.7 / 90.9 and 49.8 / 41.4 / 62.3; 3 x 150 behind up to 200, 32 x 128, 31.1 /
-//      31.1 / 36.8 and 20.4 / 20.4 / 27.6; 301 behind 150, 16 x 64, 21.7 / 21.7 / 18.9 and 16.2 /
-//      16.2 / 16.4. An explicit size is kept.
+//      ceil(context / 1024) >= 8192, else 512. A call of partitioned tiles alone takes
+//      another size of 512, 1024, 256 and 128 keys where that is estimated to take an eighth
+//      less and its workspace fits PKV_STATIC_SCRATCH_BYTES. A tile walks its keys in one serial
+//      chain, so a few long tiles have to be split to occupy 256 CUs, while a split costs each
+//      part its set-up, its rows' way through the workspace, and the reduce's launch. The
+//      estimate (see tile_partition) is fitted to 224 calls of 1 to 8 chunks at 4 to 32 heads of
+//      32 to 256 dimensions, each timed at the four sizes: the choice is 1.5% off the best size
+//      (geometric mean) and on none of them slower than the rule above alone, which is 8.4% off.
+//      Measured at 1024 / 512 / 256 / 128 keys: 64 rows behind 1000, 8 x 128 heads, float32 68.8 /
+//      40.6 / - / 20.0 us (128 taken); 301 behind 150, 16 x 64, float32, 21.7 / 21.7 / - / 18.9
+//      (128); 4 x 115 behind up to 62, 4 x 32, float32, 14.0 / 13.8 / 13.9 / 17.3 (512); 3 x 420
+//      behind up to 54, 8 x 256, bfloat16, 33.0 / 32.7 / 38.4 / 41.1 (1024); 1016 behind 1624, 8 x
+//      128, float32, 82.2 / 91.3 / 86.4 / 98.3 (1024). An explicit size is kept.
 //   5. PKV_ATTN_SHARED_KV when >= 25% of the block ids the row pass still reads repeat;
 //      PKV_ATTN_SHORT_ROWS when the row-pass items average < 256 keys; PKV_ATTN_DOMINANT_TILES
 //      when the call has both passes and the tile pass's estimated time is at least 1.1 times
@@ -62,8 +64,17 @@ constexpr int64_t kShortRowKeys = 256;
 constexpr int64_t kDominantTileWeight = 34;  // rule 5: tile_keys * 34 >= row_keys * esize * 275
 constexpr int64_t kDominantRowWeight = 275;
 constexpr int kDefaultPlanPartition = 512;
-constexpr int64_t kTargetTileItems = 200;  // rule 4: a workgroup on most of 256 CUs
-constexpr int64_t kTargetUnsplitItems = 128;
+// Rule 4's estimate, in picoseconds: a key of a tile takes kTileKeyBase + kTileKeyDim * head_dim
+// (float32, bfloat16 pools), a part's set-up as long as kTileSetupKeys keys; kTileSlots workgroups
+// run at full speed at a time; the reduce's launch and each partial row's float through the
+// workspace.
+constexpr int64_t kTileKeyBase[2] = {25000, 12000};
+constexpr int64_t kTileKeyDim[2] = {250, 160};
+constexpr int64_t kTileSlots[2] = {384, 320};
+constexpr int64_t kTileSetupKeys = 64;
+constexpr int64_t kReduceTime = 5000000;
+constexpr int64_t kPartialFloatTime = 3;
+constexpr int64_t kOtherwiseMargin = 8;  // another size must be estimated an eighth faster
 
 struct Tile {
   int32_t first, count, begin, end;
@@ -237,25 +248,44 @@ int64_t distinct_count(std::vector<int32_t>& ids) {
   return std::unique(ids.begin(), ids.end()) - ids.begin();
 }
 
-// Rule 4 for a call of partitioned tiles alone; `otherwise` when its workspace would not fit the
-// library's static scratch.
+// Rule 4 for a call of partitioned tiles alone: `otherwise`, or the size of 512, 1024, 256 and 128
+// keys that is estimated faster by the margin and keeps the workspace in the static scratch. The
+// time of a size is the longer of its longest part and all parts spread over the slots, and where a
+// tile is split the reduce.
 int32_t tile_partition(const std::vector<Tile>& tiles, const std::vector<int64_t>& vis, int32_t num_heads,
-                       int32_t head_dim, int64_t max_context, int32_t otherwise) {
+                       int32_t head_dim, int64_t max_context, bool wide_keys, int32_t otherwise) {
+  const int type = wide_keys ? 0 : 1;
   std::vector<int64_t> longest;
   longest.reserve(tiles.size());
   for (const Tile& t : tiles) {
     longest.push_back(*std::max_element(vis.begin() + t.first, vis.begin() + t.first + t.count));
   }
   const int64_t longest_of_all = *std::max_element(longest.begin(), longest.end());
-  int32_t size = 512;
-  for (; size > 128; size /= 2) {
-    int64_t items = 0;
-    for (const int64_t v : longest) items += std::max<int64_t>(1, ceil_div(v, size)) * num_heads;
-    if (items >= (longest_of_all > size ? kTargetTileItems : kTargetUnsplitItems)) break;
+  int32_t best = otherwise;
+  int64_t best_time = INT64_MAX;
+  for (const int32_t size : {otherwise, 512, 1024, 256, 128}) {
+    const int64_t parts = ceil_div(max_context, size);  // as pkv_attention_workspace_bytes counts them
+    if (size != otherwise &&
+        static_cast<int64_t>(vis.size()) * num_heads * parts * (head_dim + 2) * 4 > PKV_STATIC_SCRATCH_BYTES) {
+      continue;
+    }
+    int64_t keys = 0, partial_rows = 0;
+    for (size_t i = 0; i < tiles.size(); ++i) {
+      const int64_t n = ceil_div(longest[i], size);
+      keys += longest[i] + kTileSetupKeys * n;
+      if (n > 1) partial_rows += tiles[i].count * n;
+    }
+    const int64_t chain = std::min<int64_t>(longest_of_all, size) + kTileSetupKeys;
+    int64_t time = (kTileKeyBase[type] + kTileKeyDim[type] * head_dim) *
+                   std::max(chain, ceil_div(keys * num_heads, kTileSlots[type]));
+    if (longest_of_all > size) time += kReduceTime + kPartialFloatTime * partial_rows * num_heads * (head_dim + 2);
+    if (size == otherwise) time -= time / kOtherwiseMargin;
+    if (time < best_time) {
+      best_time = time;
+      best = size;
+    }
   }
-  const int64_t parts = ceil_div(max_context, size);  // as pkv_attention_workspace_bytes counts them
-  const int64_t bytes = static_cast<int64_t>(vis.size()) * num_heads * parts * (head_dim + 2) * 4;
-  return bytes <= PKV_STATIC_SCRATCH_BYTES ? size : otherwise;
+  return best;
 }
 
 int32_t prefix_partition(int64_t shared_tokens, int64_t tiles, int32_t num_heads) {
@@ -386,7 +416,7 @@ extern "C" int pkv_plan_batch(const int32_t* query_seq, const int32_t* query_pos
       const int64_t per_seq = std::max<int64_t>(1, num_queries / n_present);
       partition = wide * per_seq * num_heads >= kWidePartitionItems ? 1024 : 512;
       if (row_pass.empty() && tiles[0].end != PKV_TILE_WHOLE) {
-        partition = tile_partition(tiles, vis, num_heads, head_dim, max_context, partition);
+        partition = tile_partition(tiles, vis, num_heads, head_dim, max_context, kv_dtype == PKV_F32, partition);
       }
     }
   }

@@ -423,10 +423,17 @@ MIN_PREFIX_PARTITION = 256
 #: final rows written directly, nothing for the reduce) once the call has at least this many
 #: (tile, head) workgroups: four per CU of 256 keeps the chip full without splitting contexts.
 WHOLE_TILE_GROUPS = 1024
-#: (tile, head, partition) items the partition choice of a call of partitioned tiles alone aims for.
-TARGET_TILE_ITEMS = 200
-#: ... and the items that are enough where no tile spans two partitions (no reduce follows).
-TARGET_UNSPLIT_ITEMS = 128
+#: The estimate behind the partition choice of a call of partitioned tiles alone, in picoseconds
+#: (float32, bfloat16 pools): a tile's key takes TILE_KEY_BASE + TILE_KEY_DIM * head_dim, a part's
+#: set-up as long as TILE_SETUP_KEYS keys, TILE_SLOTS workgroups run at full speed at a time; then
+#: the reduce's launch and each partial row's float through the workspace.
+TILE_KEY_BASE = (25000, 12000)
+TILE_KEY_DIM = (250, 160)
+TILE_SLOTS = (384, 320)
+TILE_SETUP_KEYS = 64
+REDUCE_TIME = 5_000_000
+PARTIAL_FLOAT_TIME = 3
+OTHERWISE_MARGIN = 8  # another size must be estimated an eighth faster
 #: Tile record end partition of a whole tile (include/pkv.h PKV_TILE_WHOLE).
 TILE_WHOLE = -1
 #: Row-pass items shorter than this many keys on average launch the lighter row-pass workgroup
@@ -585,22 +592,31 @@ def _prefix_partition(shared_tokens: int, tiles: int, num_heads: int) -> int:
 
 
 def _tile_partition(
-    tiles: np.ndarray, visible: np.ndarray, num_heads: int, head_dim: int, max_context: int, otherwise: int
+    tiles: np.ndarray, visible: np.ndarray, num_heads: int, head_dim: int, max_context: int, wide_keys: bool, otherwise: int
 ) -> int:  # fmt: skip
-    """Partition size of a call of partitioned tiles alone: the largest of 512, 256 and 128 keys
-    that makes TARGET_TILE_ITEMS (tile, head, partition) items, or TARGET_UNSPLIT_ITEMS where it
-    splits no tile (and no reduce follows), or 128; ``otherwise`` when the
-    split-context workspace would not fit the library's static scratch. A tile walks its keys in
-    one serial chain, so a few tiles have to be split to fill the GPU."""
+    """Partition size of a call of partitioned tiles alone: ``otherwise``, or the one of 512, 1024,
+    256 and 128 keys that is estimated faster by the margin and whose split-context workspace fits
+    the library's static scratch. A tile walks its keys in one serial chain, so a
+    few long tiles have to be split to fill the GPU; a split costs set-up, workspace and reduce."""
+    kind = 0 if wide_keys else 1
     longest = np.fromiter((visible[f : f + c].max() for f, c in tiles[:, :2].tolist()), np.int64, tiles.shape[0])
-    size = 512
-    while size > 128:
-        items = int(np.maximum(1, -(-longest // size)).sum()) * num_heads
-        if items >= (TARGET_TILE_ITEMS if longest.max() > size else TARGET_UNSPLIT_ITEMS):
-            break
-        size //= 2
-    need = visible.size * num_heads * -(-max_context // size) * (head_dim + 2) * 4
-    return size if need <= _native.STATIC_SCRATCH_BYTES else otherwise
+    top, best, best_time = int(longest.max()), otherwise, None
+    for size in (otherwise, 512, 1024, 256, 128):
+        need = visible.size * num_heads * -(-max_context // size) * (head_dim + 2) * 4
+        if size != otherwise and need > _native.STATIC_SCRATCH_BYTES:
+            continue
+        parts = -(-longest // size)
+        keys = int((longest + TILE_SETUP_KEYS * parts).sum())
+        chain = min(top, size) + TILE_SETUP_KEYS
+        time = (TILE_KEY_BASE[kind] + TILE_KEY_DIM[kind] * head_dim) * max(chain, -(-keys * num_heads // TILE_SLOTS[kind]))
+        if top > size:
+            partial_rows = int((tiles[:, 1] * parts)[parts > 1].sum())
+            time += REDUCE_TIME + PARTIAL_FLOAT_TIME * partial_rows * num_heads * (head_dim + 2)
+        if size == otherwise:
+            time -= time // OTHERWISE_MARGIN
+        if best_time is None or time < best_time:
+            best, best_time = size, time
+    return best
 
 
 def _visible(seq: np.ndarray, contexts: np.ndarray, positions: np.ndarray | None) -> np.ndarray:
@@ -760,7 +776,8 @@ def plan_batch(
         if partition == 0:
             partition = _wide_partition(contexts[present], num_heads, max(1, seq.size // present.size))
             if rows.size == 0 and tiles[0, 3] != TILE_WHOLE:
-                partition = _tile_partition(tiles, visible, num_heads, head_dim, int(contexts[present].max()), partition)
+                partition = _tile_partition(tiles, visible, num_heads, head_dim, int(contexts[present].max()),
+                                            kv_dtype == torch.float32, partition)  # fmt: skip
     prefix_tiles = []
     for start, count, common in groups:
         parts = common * block_size // partition

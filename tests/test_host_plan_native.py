@@ -164,23 +164,25 @@ def test_small_buffers_grow_and_bad_arguments_are_refused() -> None:
 @pytest.mark.parametrize(
     ("chunks", "heads", "dim", "want"),
     [
-        ([(8, 0)], 1, 64, 128),  # one short tile: nothing to split, the smallest size
-        ([(64, 0)], 128, 32, 512), ([(64, 0)], 127, 32, 128),  # 128 items as they are, and 127
-        ([(64, 500)], 100, 32, 512), ([(64, 500)], 99, 32, 256),  # 200 items of two partitions, and 198
-        ([(301, 150)], 16, 64, 128), ([(1000, 0)], 12, 64, 512), ([(301, 1500)], 32, 128, 512),
-        ([(64, 1024)], 64, 32, 256), ([(64, 20_000)], 22, 32, 512), ([(1000, 30_000)], 1, 256, 512),
-        # 512 keys would make the items, but 130 MB of workspace: the size such a call had before
-        ([(64, 29_936), (1000, 0)], 4, 128, 1024),
+        ([(8, 0)], 1, 64, (512, 512)), ([(64, 64)], 8, 32, (512, 512)),  # shorter than any split pays for
+        ([(64, 0)], 127, 32, (512, 512)), ([(137, 192), (137, 0), (137, 90)], 8, 32, (512, 512)),
+        ([(301, 150)], 16, 64, (128, 512)), ([(64, 500)], 99, 32, (128, 1024)), ([(1000, 0)], 12, 64, (256, 256)),
+        ([(64, 1000)], 8, 128, (128, 128)), ([(64, 1024)], 64, 32, (256, 256)),  # few long tiles
+        ([(420, 54)] * 3, 8, 256, (1024, 1024)), ([(301, 1500)], 32, 128, (1024, 1024)),  # enough items whole
+        ([(1016, 1624)], 8, 128, (1024, 1024)), ([(1000, 30_000)], 1, 256, (1024, 1024)),
+        # a smaller size would not fit the static scratch; 1024 itself does not in the last
+        ([(64, 29_936), (1000, 0)], 4, 128, (1024, 1024)), ([(64, 60_000), (1000, 0)], 8, 256, (1024, 1024)),
     ],
 )  # fmt: skip
 def test_partition_of_calls_of_tiles_alone(chunks, heads, dim, want) -> None:
-    """The largest of 512, 256 and 128 keys that makes 200 (tile, head, partition) items (128
-    where no tile spans two partitions), or 128; and only sizes whose workspace fits the library's static scratch."""
+    """With float32 and bfloat16 pools: a size whose workspace fits the library's static scratch
+    where it is estimated an eighth faster than the general rule's; both planners alike."""
     contexts = np.asarray([offset + rows for rows, offset in chunks])
     positions = np.concatenate([np.arange(offset, offset + rows) for rows, offset in chunks])
     seq = np.repeat(np.arange(len(chunks)), [rows for rows, _ in chunks])
     tables = [np.arange(-(-int(c) // 16)) for c in contexts]
-    python = ops.plan_batch(seq, dim, heads, tables, contexts, 16, query_positions=positions)
-    native = ops.plan_batch_native(seq, dim, heads, tables, contexts, 16, query_positions=positions)
-    _same(python, native)
-    assert native.partition_size == want and native.rows.shape[0] == 0
+    for dtype, size in zip((torch.float32, torch.bfloat16), want):
+        python = ops.plan_batch(seq, dim, heads, tables, contexts, 16, query_positions=positions, kv_dtype=dtype)
+        native = ops.plan_batch_native(seq, dim, heads, tables, contexts, 16, query_positions=positions, kv_dtype=dtype)
+        _same(python, native)
+        assert native.partition_size == size and native.rows.shape[0] == 0
