@@ -1053,7 +1053,7 @@ struct SplitShape {
   static constexpr int kVRow = D + (D % 128 == 0 ? 16 : D % 64 == 0 ? 48 : 16);
   static constexpr int kKTile = kKeys * kKRow;  // one plane
   static constexpr int kVTile = kKeys * kVRow;
-  static constexpr int kElems = kPlanes * (kKTile + kVTile);  // K planes, then V planes  // K planes, then V planes
+  static constexpr int kElems = kPlanes * (kKTile + kVTile);  // K planes, then V planes
 };
 
 // One work item of the tile pass (numbered as tile_item's). Returns true, with nothing written,
@@ -1068,9 +1068,10 @@ struct SplitShape {
 // wavefronts with 64), which the pinned order below is for. Measured on MI355X, 8 chunks of 512
 // rows at offsets up to 2048, 32 x 128 heads (86 GFLOP), same boxes: bfloat16 pools 0.685 ms with
 // float32 products, 0.250 with these unordered, 0.235 ordered; float32 pools 0.70, 0.505 and
-// 0.49; one chunk of 301 rows with 16 x 64 heads 29.6, 26.1 and 21.6 us. Relative error against
-// float64: 4.9e-7 (bfloat16) and 6.9e-7, 7.7e-7 with the float32 products, whose longer chains of
-// 4-term sums round more often.
+// 0.49; one chunk of 301 rows with 16 x 64 heads 29.6, 26.1 and 21.6 us. (Through the public call on
+// slower boxes 0.76-0.82 -> 0.27-0.28 and 0.78-0.85 -> 0.58-0.61 ms.) Relative error against
+// float64 there: 3.6e-7 (bfloat16) and 5.0e-7, 6.0e-7 with the float32 products, whose longer
+// chains of 4-term sums round more often.
 template <typename KVT, int D, bool kPow2Block>
 __device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, uint32_t tid, int* s_table,
                                                 uint16_t* s_kv, int* s_vis) {

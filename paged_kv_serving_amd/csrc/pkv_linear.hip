@@ -1,7 +1,7 @@
 // The matrix products of a small decoder with the row-wise steps around them in one launch each:
 // RMSNorm of the input rows before the product, and after it the residual add, RoPE with the
-// slot-mapped append, or the SwiGLU gate. At the sizes this serves (up to 512 rows of at most 512
-// floats) every launch is latency: a library product takes 4.5-6.7 us, a norm 3.2, RoPE + append
+// slot-mapped append, or the SwiGLU gate. At the sizes this serves (up to 512 rows, d_model up
+// to 256) every launch is latency: a library product takes 4.5-6.7 us, a norm 3.2, RoPE + append
 // 3.8, a gate 2.7, whatever they compute, and a layer had nine of them.
 //
 // Products are float32 (v_mfma_f32_16x16x4f32). One workgroup computes 16 rows x 64 columns, a
