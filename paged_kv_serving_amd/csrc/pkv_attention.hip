@@ -18,7 +18,7 @@
 //     wavefronts of 16 queries each; the scores are computed as S^T = K Q^T and the output as
 //     O^T = V^T P^T, so every lane owns eight scores of one query per 32 keys and the P operand
 //     of the second product is the lane's own registers. The products run on
-//     v_mfma_f32_16x16x32_bf16 over exact bfloat16 pieces of the float32 operands; float32
+//     v_mfma_f32_16x16x32_bf16 over bfloat16 pieces of the float32 operands; float32
 //     products (v_mfma_f32_16x16x4f32) remain for tiles that meet an infinity or NaN and for
 //     float32 tiles beside the lean row pass.
 //  3. reduce: rows whose visible context spans several partitions merge the per-partition
@@ -1003,26 +1003,41 @@ __device__ __forceinline__ void tile_item(const Params& a, uint32_t bid, uint32_
 }
 
 // ---------------------------------------------------------------------------------------------
-// Tile items on bf16 MFMA with exact three-way splits. A float32 x is hi + mid + lo, each the next
-// 8 significant bits of x as a bfloat16 (truncated, so hi never overflows and the sum is exactly x
-// down to the subnormals); a product of two bfloat16 values is exact in float32 and the matrix
-// core accumulates in float32. With bfloat16 pools K and V are one piece, so an exact q * k or
-// p * v takes 3 products; with float32 pools the 6 products of weight >= 2^-16 are kept (the
-// dropped ones are below 2^-23 of the product). v_mfma_f32_16x16x32_bf16 does 16 times the work of
-// v_mfma_f32_16x16x4f32 per cycle, so the products cost 3/16 or 6/16 of the float32 ones.
+// Tile items on bf16 MFMA with three-way splits. A float32 x is hi + mid + lo, each the next 8
+// significant bits of x as a bfloat16, so the sum is exactly x (its bits from 2^-133 up). A product
+// of two bfloat16 values is exact in float32 and the matrix core accumulates in float32.
+// With bfloat16 pools K and V are one piece, so q * k or p * v takes 3 products and loses nothing;
+// the pieces of q and p are cut off there (15 registers spilled instead of 11 at head_dim 128 with
+// rounded ones). With float32 pools 6 of the 9 products are computed and the pieces are rounded to
+// nearest: |mid| <= 2^-8 |x| and |lo| <= 2^-17 |x| with either sign, so the three products left out
+// (mid * lo twice, lo * lo) are together at most 2^-24 of the product, the size of one float32
+// rounding, and of either sign. (Pieces cut off would leave out up to 2^-21, always towards zero.)
+// v_mfma_f32_16x16x32_bf16 does 16 times the work of v_mfma_f32_16x16x4f32 per cycle, so the
+// products cost 3/16 or 6/16 of the float32 ones.
 // ---------------------------------------------------------------------------------------------
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
-// The next piece of two floats, packed as a bfloat16 pair (x0 in the low half); x0 and x1 become
-// what is left of them.
+// The next piece of two floats, rounded to nearest (a value that rounds to a bfloat16 infinity then
+// goes the way of infinities) or cut off, packed as a bfloat16 pair (x0 in the low half); x0 and x1
+// become what is left of them.
+template <bool kNearest>
 __device__ __forceinline__ uint32_t take_piece(float& x0, float& x1) {
+  if constexpr (kNearest) {
+    const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{x0, x1}), bf16x2));
+    x0 -= bf16_lo(pair);
+    x1 -= bf16_hi(pair);
+    return pair;
+  }
   const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
   x0 -= __uint_as_float(u0 & 0xffff0000u);
   x1 -= __uint_as_float(u1 & 0xffff0000u);
   return __builtin_amdgcn_perm(u1, u0, 0x07060302u);
 }
+// What is left after two pieces has at most 8 significant bits: it is its own bfloat16.
 __device__ __forceinline__ uint32_t last_piece(float x0, float x1) {
   return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
 }
@@ -1069,9 +1084,11 @@ struct SplitShape {
 // rows at offsets up to 2048, 32 x 128 heads (86 GFLOP), same boxes: bfloat16 pools 0.685 ms with
 // float32 products, 0.250 with these unordered, 0.235 ordered; float32 pools 0.70, 0.505 and
 // 0.49; one chunk of 301 rows with 16 x 64 heads 29.6, 26.1 and 21.6 us. (Through the public call on
-// slower boxes 0.76-0.82 -> 0.27-0.28 and 0.78-0.85 -> 0.58-0.61 ms.) Relative error against
-// float64 there: 3.6e-7 (bfloat16) and 5.0e-7, 6.0e-7 with the float32 products, whose longer
-// chains of 4-term sums round more often.
+// slower boxes 0.76-0.82 -> 0.27-0.28 and 0.78-0.85 -> 0.58-0.61 ms.) The rounded pieces of float32
+// pools take 588 us there and 18.9 us for one chunk of 301 rows where cut-off ones took 584 and 18.5.
+// Relative error against float64, 8 chunks: 4.0e-7 (bfloat16) and 5.5e-7 (float32; 5.6e-7 with
+// cut-off pieces, 6.6e-7 with the float32 products, whose longer chains of 4-term sums round more
+// often); the 301-row chunk 2.3e-7 (2.6e-7 with cut-off pieces).
 template <typename KVT, int D, bool kPow2Block>
 __device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, uint32_t tid, int* s_table,
                                                 uint16_t* s_kv, int* s_vis) {
@@ -1136,8 +1153,8 @@ __device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, u
       for (int e = 0; e < 8; ++e) raw[e] = q_ok ? raw[e] * a.scale_log2 : 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        qp[0][s][e] = take_piece(raw[2 * e], raw[2 * e + 1]);
-        qp[1][s][e] = take_piece(raw[2 * e], raw[2 * e + 1]);
+        qp[0][s][e] = take_piece<kF32>(raw[2 * e], raw[2 * e + 1]);
+        qp[1][s][e] = take_piece<kF32>(raw[2 * e], raw[2 * e + 1]);
         qp[2][s][e] = last_piece(raw[2 * e], raw[2 * e + 1]);
       }
     }
@@ -1244,13 +1261,13 @@ __device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, u
         const int e = step / 2;  // pair of the chunk
         float x0 = __uint_as_float(raw[u][e / 2][2 * (e % 2)]), x1 = __uint_as_float(raw[u][e / 2][2 * (e % 2) + 1]);
         if (step % 2 == 0) {
-          uint32_t hi = take_piece(x0, x1);
+          uint32_t hi = take_piece<kF32>(x0, x1);
           pin(hi);
           pl[0][e] = hi;
           raw[u][e / 2][2 * (e % 2)] = __float_as_uint(x0);
           raw[u][e / 2][2 * (e % 2) + 1] = __float_as_uint(x1);
         } else {
-          uint32_t mid = take_piece(x0, x1);
+          uint32_t mid = take_piece<kF32>(x0, x1);
           uint32_t lo = last_piece(x0, x1);
           pin(lo);
           pl[1][e] = mid;
@@ -1385,11 +1402,11 @@ __device__ __forceinline__ bool tile_item_split(const Params& a, uint32_t bid, u
       l_part += p1;
       pin(l_part);
     } else if (task % 3 == 1) {
-      uint32_t hi = take_piece(p0, p1);
+      uint32_t hi = take_piece<kF32>(p0, p1);
       pin(hi);
       pp[0][e] = hi;
     } else {
-      uint32_t mid = take_piece(p0, p1);
+      uint32_t mid = take_piece<kF32>(p0, p1);
       uint32_t lo = last_piece(p0, p1);
       pin(lo);
       pp[1][e] = mid;

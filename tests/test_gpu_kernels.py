@@ -1231,3 +1231,36 @@ def test_tiles_with_infinite_values_fall_back_to_float32_products(device, kv, di
             clean = np.ones(got.shape, bool)
             clean[first:, :, 1] = False
             assert np.max(np.abs(np.where(clean, got, 0) - np.where(clean, want, 0))) < FP32_TOL, (rows, end)
+
+
+@pytest.mark.parametrize("dim", [32, 64, 128, 256])
+def test_float32_tile_products_keep_float32_precision(device, dim) -> None:
+    """Float32 tiles multiply bfloat16 pieces and leave the smallest products out, which must cost
+    no more than a float32 rounding. Operands whose low 16 significant bits are all ones leave out
+    the most (2^-21 of the product if the pieces are cut off instead of rounded). One product a * b
+    is a score of base-2 size s against a score of 0; the weight 1 / (2^s + 1) moves by s ln 2 times
+    the product's relative error, of which three float32 roundings are allowed (the part left out,
+    the product's last sum, the subtraction of the reference), plus 2^-21 for the exponential, the
+    sum of weights and the quotient."""
+    say("float32 tile products", dim)
+    rng = np.random.default_rng(dim)
+    heads, rows, block = 16, 64, 16
+
+    def full(*shape):  # random leading bits, the low 16 significant bits all ones, 4 <= value < 8
+        return (rng.integers(0x4080, 0x4100, shape).astype(np.uint32) << np.uint32(16) | np.uint32(0xFFFF)).view(np.float32)
+
+    q = np.zeros((rows, heads, dim), np.float32)
+    keys, values = (np.zeros((1, block, heads, dim), np.float32) for _ in range(2))
+    q[:, :, 0], keys[0, 0, :, 0], values[0, 1] = full(rows, heads), full(heads), 1.0
+    q[0, :, 0] = keys[0, 0, :, 0] = np.uint32(0x4080FFFF).view(np.float32)
+    s = q[:, :, 0].astype(np.float64) * keys[0, 0, :, 0]
+    want = 1.0 / (2.0**s + 1.0)
+    to = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    for end in (0, ops.TILE_WHOLE):
+        got = ops.paged_attention_ragged(
+            to(q), to(np.ones(rows, np.int32)), to(np.zeros(rows, np.int32)), to(keys), to(values),
+            to(np.zeros((1, 1), np.int32)), to(np.asarray([2], np.int32)), float(np.log(2.0)), max_context_len=2,
+            plan=ops.upload_plan(np.zeros((0, 2), np.int32), np.asarray([[0, rows, 0, end]], np.int32), device),
+        ).cpu().numpy()[:, :, dim - 1].astype(np.float64)  # fmt: skip
+        error = np.abs(got / want - 1.0)
+        assert np.all(error <= 3 * 2.0**-24 * s * np.log(2.0) + 2.0**-21), float((error / s).max())
