@@ -53,6 +53,11 @@ typedef enum pkv_dtype {
                                     row workgroups fill in around them) instead of one
                                     (float32) or two */
 
+#define PKV_ATTN_WIDER_512 8   /* plans of tiles alone: partition_size was chosen below 512 or */
+#define PKV_ATTN_WIDER_1024 16 /* 1024 keys for speed, and the plan is as good at that size: the
+                                  call takes it where the workspace at partition_size would not
+                                  fit PKV_STATIC_SCRATCH_BYTES or the workspace given */
+
 /* pkv_paged_attention tile record: end partition of a tile computed whole by one workgroup. */
 #define PKV_TILE_WHOLE (-1)
 
@@ -237,10 +242,13 @@ int pkv_tile_head_dim_supported(int32_t head_dim);
  *   partition_size   : keys per split-context partition, a positive multiple of 16, <= 1024;
  *                      0 selects the library default (512).
  *   flags            : PKV_ATTN_SHARED_KV, PKV_ATTN_SHORT_ROWS and/or PKV_ATTN_DOMINANT_TILES,
- *                      or 0. They only choose how the kernels run; the results agree within
- *                      float32 rounding (PKV_ATTN_DOMINANT_TILES: bit for bit).
+ *                      or 0, and one of PKV_ATTN_WIDER_512 and PKV_ATTN_WIDER_1024 (which need a
+ *                      plan without rows, whose tiles all run through their last partition). They
+ *                      only choose how the kernels run; the results agree within float32 rounding
+ *                      (PKV_ATTN_DOMINANT_TILES: bit for bit).
  *   workspace        : float32 scratch of pkv_attention_workspace_bytes(...) bytes (may be
- *                      NULL when that is 0); 16-byte aligned when num_tiles > 0.
+ *                      NULL when that is 0); 16-byte aligned when num_tiles > 0. With
+ *                      PKV_ATTN_WIDER_*, that size's bytes are enough.
  * A query whose every key is masked gets a zero output (attention.py:120-121).
  * Block ids are read only for positions below the query's visible length, so table entries
  * past a sequence's last used block may hold anything. A block id outside [0, num_blocks) at a
@@ -270,8 +278,8 @@ int pkv_paged_attention(float* out, const float* queries, int64_t query_token_st
  * (64 MiB) in the library, one copy per GPU, held until the process ends. The call allocates
  * nothing and creates nothing: on a device's first use it only looks up that device's copy of
  * the array (pkv_init does the same). A batch whose workspace
- * (pkv_attention_workspace_bytes) exceeds the buffer is refused with PKV_ETOOBIG before anything
- * is enqueued. Nothing in the buffer needs to start at zero: every entry a call reads, the same
+ * (pkv_attention_workspace_bytes, with PKV_ATTN_WIDER_* at the wider size) exceeds the buffer is
+ * refused with PKV_ETOOBIG before anything is enqueued. Nothing in the buffer needs to start at zero: every entry a call reads, the same
  * call has written before. Every call on one GPU shares that GPU's buffer, so two calls whose
  * execution overlaps on one GPU (on different streams, without ordering between them) race;
  * calls on one stream, or ordered by events, do not.
@@ -347,9 +355,12 @@ int pkv_paged_attention_append(
  *   context_lens               : int32 [num_seqs], host.
  *   kv_dtype                   : the pools' element type; it weighs the row pass's bytes
  *                                against the tile pass's products for PKV_ATTN_DOMINANT_TILES.
- *   partition_size             : 0 lets the planner choose (for calls of tiles alone, within the
- *                                static scratch at the longest present context: pass that as
- *                                max_context_len); a positive value is kept.
+ *   partition_size             : 0 lets the planner choose; a positive value is kept. For calls
+ *                                of tiles alone the choice may be below 512 keys where that is
+ *                                faster and its workspace at the longest present context fits
+ *                                the static scratch; flags then name the wider size
+ *                                (PKV_ATTN_WIDER_*) that a call with a larger max_context_len
+ *                                takes instead.
  *   min_tile_rows              : the shortest run of one sequence's rows made into tiles (8).
  *   rows_out [rows_capacity, 2], tiles_out [tiles_capacity, 4], merge_out [merge_capacity] :
  *                                int32 outputs in pkv_paged_attention's layout.

@@ -65,6 +65,8 @@ PKV_BF16 = 1
 PKV_ATTN_SHARED_KV = 1
 PKV_ATTN_SHORT_ROWS = 2
 PKV_ATTN_DOMINANT_TILES = 4
+PKV_ATTN_WIDER_512 = 8
+PKV_ATTN_WIDER_1024 = 16
 PKV_TILE_WHOLE = -1
 
 PKV_OK = 0

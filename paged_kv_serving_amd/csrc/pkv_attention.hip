@@ -33,6 +33,7 @@
 // visible block are never read.
 #include <math.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1869,6 +1870,21 @@ int64_t parts_for(int32_t max_context_len, int part) {
   return (static_cast<int64_t>(max_context_len) + part - 1) / part;
 }
 
+constexpr int kWiderFlags = PKV_ATTN_WIDER_512 | PKV_ATTN_WIDER_1024;
+
+// The partition size of a call whose workspace may take `available` bytes: with a PKV_ATTN_WIDER_*
+// flag the wider size where the plan's own would need more than that or than the static scratch.
+// (The planner bounds its choice by the contexts it sees. A caller's max_context_len may be larger,
+// and the call must then neither be refused nor take several times the memory.)
+int call_partition(int32_t partition_size, int32_t flags, int64_t num_queries, int32_t num_heads, int32_t head_dim,
+                   int32_t max_context_len, int64_t available) {
+  const int part = resolve_partition(partition_size);
+  const int wider = flags & PKV_ATTN_WIDER_512 ? 512 : flags & PKV_ATTN_WIDER_1024 ? 1024 : 0;
+  if (part < 0 || part >= wider) return part;
+  const int64_t need = pkv_attention_workspace_bytes(num_queries, num_heads, head_dim, max_context_len, part);
+  return need > std::min<int64_t>(available, PKV_STATIC_SCRATCH_BYTES) ? wider : part;
+}
+
 }  // namespace
 }  // namespace pkv
 
@@ -1945,9 +1961,11 @@ int attention_call(float* out, const float* queries, int64_t query_token_stride,
                    int32_t head_dim, float scale, int32_t max_context_len, int32_t partition_size,
                    int32_t flags, float* workspace, int64_t workspace_bytes, int device,
                    void* stream, const AppendSource* append) {
-  const int part = resolve_partition(partition_size);
+  if (flags & ~(PKV_ATTN_SHARED_KV | PKV_ATTN_SHORT_ROWS | PKV_ATTN_DOMINANT_TILES | kWiderFlags)) return PKV_EINVAL;
+  if ((flags & kWiderFlags) == kWiderFlags) return PKV_EINVAL;
+  const int part = call_partition(partition_size, flags, num_queries, num_heads, head_dim, max_context_len,
+                                  workspace ? workspace_bytes : 0);
   if (part < 0) return PKV_EINVAL;
-  if (flags & ~(PKV_ATTN_SHARED_KV | PKV_ATTN_SHORT_ROWS | PKV_ATTN_DOMINANT_TILES)) return PKV_EINVAL;
   const bool stream_kv = (flags & PKV_ATTN_SHARED_KV) == 0;
   if (num_queries < 0 || num_rows < 0 || num_tiles < 0 || num_merge_rows < -1 || num_blocks < 1 ||
       block_size < 1 ||
@@ -1975,6 +1993,7 @@ int attention_call(float* out, const float* queries, int64_t query_token_stride,
       (num_merge_rows > 0 && !merge_rows)) {
     return PKV_EINVAL;
   }
+  if ((flags & kWiderFlags) && (num_rows > 0 || num_tiles == 0)) return PKV_EINVAL;
   if (num_tiles > 0 && !pkv_tile_head_dim_supported(head_dim)) return PKV_EUNSUPPORTED;
   const int64_t parts = parts_for(max_context_len, part);
   if (parts > 0x7fffffff) return PKV_EUNSUPPORTED;
@@ -2102,8 +2121,10 @@ extern "C" int pkv_paged_attention_noalloc(
     void* stream) {
   using namespace pkv;
   if (device < 0 || device >= kMaxDevices) return PKV_EINVAL;
-  const int64_t need = pkv_attention_workspace_bytes(num_queries, num_heads, head_dim,
-                                                     max_context_len, partition_size);
+  const int part = call_partition(partition_size, flags, num_queries, num_heads, head_dim, max_context_len,
+                                  PKV_STATIC_SCRATCH_BYTES);
+  const int64_t need = part < 0 ? -1 : pkv_attention_workspace_bytes(num_queries, num_heads, head_dim,
+                                                                     max_context_len, part);
   if (need < 0) return PKV_EINVAL;
   if (need > PKV_STATIC_SCRATCH_BYTES) return PKV_ETOOBIG;
   float* workspace = nullptr;

@@ -21,7 +21,8 @@
 //      prefix with about 512 tile workgroups; without groups 1024 when rows x heads x
 //      ceil(context / 1024) >= 8192, else 512. A call of partitioned tiles alone takes
 //      another size of 512, 1024, 256 and 128 keys where that is estimated to take an eighth
-//      less and its workspace fits PKV_STATIC_SCRATCH_BYTES. A tile walks its keys in one serial
+//      less and its workspace fits PKV_STATIC_SCRATCH_BYTES; a size below the rule's carries
+//      the rule's in PKV_ATTN_WIDER_*, for calls with a larger max_context_len. A tile walks its keys in one serial
 //      chain, so a few long tiles have to be split to occupy 256 CUs, while a split costs each
 //      part its set-up, its rows' way through the workspace, and the reduce's launch. The
 //      estimate (see tile_partition) is fitted to 224 calls of 1 to 8 chunks at 4 to 32 heads of
@@ -395,6 +396,7 @@ extern "C" int pkv_plan_batch(const int32_t* query_seq, const int32_t* query_pos
 
   // Rule 4: the partition size.
   int32_t partition = partition_size;
+  int32_t wider = 0;  // PKV_ATTN_WIDER_* when the partition size is smaller than it would be without the estimate
   if (partition == 0) {
     if (!groups.empty()) {
       const Group* largest = &groups[0];
@@ -416,7 +418,9 @@ extern "C" int pkv_plan_batch(const int32_t* query_seq, const int32_t* query_pos
       const int64_t per_seq = std::max<int64_t>(1, num_queries / n_present);
       partition = wide * per_seq * num_heads >= kWidePartitionItems ? 1024 : 512;
       if (row_pass.empty() && tiles[0].end != PKV_TILE_WHOLE) {
-        partition = tile_partition(tiles, vis, num_heads, head_dim, max_context, kv_dtype == PKV_F32, partition);
+        const int32_t otherwise = partition;
+        partition = tile_partition(tiles, vis, num_heads, head_dim, max_context, kv_dtype == PKV_F32, otherwise);
+        if (partition < otherwise) wider = otherwise == 512 ? PKV_ATTN_WIDER_512 : PKV_ATTN_WIDER_1024;
       }
     }
   }
@@ -581,6 +585,6 @@ extern "C" int pkv_plan_batch(const int32_t* query_seq, const int32_t* query_pos
                         tile_keys * kDominantTileWeight >= key_sum * esize * kDominantRowWeight;
   launch_out[0] = partition;
   launch_out[1] = (shared_kv ? PKV_ATTN_SHARED_KV : 0) | (short_rows ? PKV_ATTN_SHORT_ROWS : 0) |
-                  (dominant ? PKV_ATTN_DOMINANT_TILES : 0);
+                  (dominant ? PKV_ATTN_DOMINANT_TILES : 0) | wider;
   return PKV_OK;
 }

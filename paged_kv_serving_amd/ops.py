@@ -351,7 +351,9 @@ class AttentionPlan:
     merges (None: every row, which is only correct without whole tiles). ``partition_size``
     (0: library default), ``shared_kv``, ``short_rows`` (the lighter row-pass workgroup for
     short items) and ``dominant_tiles`` (three tile-pass workgroups per CU beside the rows)
-    choose the launch.
+    choose the launch. ``wider_partition`` (512, 1024 or 0; plans of tiles alone): the size a call
+    takes instead where the workspace at ``partition_size`` and its ``max_context_len`` would not
+    fit the library's static scratch.
     """
 
     rows: torch.Tensor
@@ -361,6 +363,7 @@ class AttentionPlan:
     merge: torch.Tensor | None = None
     short_rows: bool = False
     dominant_tiles: bool = False
+    wider_partition: int = 0
 
     @property
     def num_rows(self) -> int:
@@ -496,6 +499,7 @@ class BatchPlan:
     merge: np.ndarray | None = None
     short_rows: bool = False
     dominant_tiles: bool = False
+    wider_partition: int = 0
 
 
 def _padded_tables(tables, sid: np.ndarray, used: np.ndarray, width: int) -> np.ndarray:
@@ -595,8 +599,8 @@ def _tile_partition(
     tiles: np.ndarray, visible: np.ndarray, num_heads: int, head_dim: int, max_context: int, wide_keys: bool, otherwise: int
 ) -> int:  # fmt: skip
     """Partition size of a call of partitioned tiles alone: ``otherwise``, or the one of 512, 1024,
-    256 and 128 keys that is estimated faster by the margin and whose split-context workspace fits
-    the library's static scratch. A tile walks its keys in one serial chain, so a
+    256 and 128 keys that is estimated faster by the margin and whose split-context workspace at
+    the longest present context fits the library's static scratch. A tile walks its keys in one serial chain, so a
     few long tiles have to be split to fill the GPU; a split costs set-up, workspace and reduce."""
     kind = 0 if wide_keys else 1
     longest = np.fromiter((visible[f : f + c].max() for f, c in tiles[:, :2].tolist()), np.int64, tiles.shape[0])
@@ -768,6 +772,7 @@ def plan_batch(
                                 padded)  # fmt: skip
     present = np.unique(seq)
     partition = partition_size
+    wider = 0
     if partition == 0:
         if groups:
             largest = max(groups, key=lambda g: g[1] * g[2])
@@ -776,8 +781,10 @@ def plan_batch(
         if partition == 0:
             partition = _wide_partition(contexts[present], num_heads, max(1, seq.size // present.size))
             if rows.size == 0 and tiles[0, 3] != TILE_WHOLE:
+                otherwise = partition
                 partition = _tile_partition(tiles, visible, num_heads, head_dim, int(contexts[present].max()),
-                                            kv_dtype == torch.float32, partition)  # fmt: skip
+                                            kv_dtype == torch.float32, otherwise)  # fmt: skip
+                wider = otherwise if partition < otherwise else 0
     prefix_tiles = []
     for start, count, common in groups:
         parts = common * block_size // partition
@@ -817,7 +824,7 @@ def plan_batch(
         keys = np.maximum(np.minimum(partition, visible[items[:, 0]] - items[:, 1].astype(np.int64) * partition), 0)
         short = bool(np.mean(keys) < SHORT_ROW_KEYS)
         dominant = _dominant_tiles(tiles, visible, int(partition), int(keys.sum()), kv_dtype_size(kv_dtype))
-    return BatchPlan(items, tiles, int(partition), _repeated_fraction_reached(ids), merge, short, dominant)
+    return BatchPlan(items, tiles, int(partition), _repeated_fraction_reached(ids), merge, short, dominant, wider)
 
 
 #: The dominant-tiles hint: a call with both passes sets it when the tile pass's estimated time
@@ -927,6 +934,7 @@ class NativePlanner:
             self._rows[:rows].copy(), self._tiles[:tiles].copy(), partition,
             bool(flags & _native.PKV_ATTN_SHARED_KV), self._merge[:merge].copy(),
             bool(flags & _native.PKV_ATTN_SHORT_ROWS), bool(flags & _native.PKV_ATTN_DOMINANT_TILES),
+            wider_partition_of(flags),
         )  # fmt: skip
 
 
@@ -942,6 +950,15 @@ def plan_batch_native(query_seq, head_dim, num_heads, tables, context_lens, bloc
     return NativePlanner().plan(query_seq, head_dim, num_heads, tables, context_lens, block_size, **kwargs)
 
 
+#: The flag of each ``wider_partition``.
+_WIDER_FLAGS = {512: _native.PKV_ATTN_WIDER_512, 1024: _native.PKV_ATTN_WIDER_1024}
+
+
+def wider_partition_of(flags: int) -> int:
+    """The wider partition size that a plan's flags name (0: none)."""
+    return next((size for size, flag in _WIDER_FLAGS.items() if flags & flag), 0)
+
+
 def _plan_flags(plan: AttentionPlan | None, shared_kv: bool) -> int:
     """pkv_paged_attention flags of a call with ``plan``."""
     flags = _native.PKV_ATTN_SHARED_KV if shared_kv else 0
@@ -949,6 +966,8 @@ def _plan_flags(plan: AttentionPlan | None, shared_kv: bool) -> int:
         flags |= _native.PKV_ATTN_SHORT_ROWS
     if plan is not None and plan.dominant_tiles:
         flags |= _native.PKV_ATTN_DOMINANT_TILES
+    if plan is not None and plan.wider_partition:
+        flags |= _WIDER_FLAGS[plan.wider_partition]
     return flags
 
 
@@ -1001,7 +1020,7 @@ def launch_paged_attention(
 def upload_plan(
     rows: np.ndarray, tiles: np.ndarray, device: torch.device, *, partition_size: int = 0,
     shared_kv: bool = False, merge: np.ndarray | None = None, short_rows: bool = False,
-    dominant_tiles: bool = False,
+    dominant_tiles: bool = False, wider_partition: int = 0,
 ) -> AttentionPlan:
     """Copy a host plan (``rows [R, 2]``, ``tiles [n, 4]``, ``merge [M]``) to the device in one
     transfer. Without a merge list, one is derived when a tile is whole (every row no whole tile
@@ -1020,14 +1039,14 @@ def upload_plan(
         rows=data[: rows.size].view(-1, 2), tiles=data[rows.size : end_tiles].view(-1, 4),
         partition_size=partition_size, shared_kv=shared_kv,
         merge=None if merge is None else data[end_tiles:], short_rows=short_rows,
-        dominant_tiles=dominant_tiles,
+        dominant_tiles=dominant_tiles, wider_partition=wider_partition,
     )  # fmt: skip
 
 
 def upload_batch_plan(plan: BatchPlan, device: torch.device) -> AttentionPlan:
     return upload_plan(plan.rows, plan.tiles, device, partition_size=plan.partition_size,
                        shared_kv=plan.shared_kv, merge=plan.merge, short_rows=plan.short_rows,
-                       dominant_tiles=plan.dominant_tiles)  # fmt: skip
+                       dominant_tiles=plan.dominant_tiles, wider_partition=plan.wider_partition)  # fmt: skip
 
 
 def attention_workspace_bytes(
@@ -1134,6 +1153,8 @@ def paged_attention_ragged(
     if shared_kv is None:
         shared_kv = plan.shared_kv if plan is not None else False
     need = attention_workspace_bytes(num_queries, heads, dim, max_context_len, partition_size)
+    if need > _native.STATIC_SCRATCH_BYTES and plan is not None and plan.wider_partition:
+        need = attention_workspace_bytes(num_queries, heads, dim, max_context_len, plan.wider_partition)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need // 4, dtype=torch.float32, device=queries.device)
     ws_ptr = workspace.data_ptr() if need else None

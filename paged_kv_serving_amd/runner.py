@@ -385,6 +385,7 @@ class ModelRunner:
         return ops.BatchPlan(
             plan_rows, plan_tiles, partition, bool(flags & _native.PKV_ATTN_SHARED_KV), merge,
             bool(flags & _native.PKV_ATTN_SHORT_ROWS), bool(flags & _native.PKV_ATTN_DOMINANT_TILES),
+            ops.wider_partition_of(flags),
         )  # fmt: skip
 
     # --- pool ---------------------------------------------------------------------------

@@ -18,8 +18,8 @@ def _same(a: ops.BatchPlan, b: ops.BatchPlan) -> None:
     assert np.array_equal(np.asarray(a.rows, np.int32).reshape(-1, 2), b.rows), "rows"
     assert np.array_equal(np.asarray(a.tiles, np.int32).reshape(-1, 4), b.tiles), "tiles"
     assert np.array_equal(np.asarray(a.merge, np.int32), b.merge), "merge"
-    assert (a.partition_size, a.shared_kv, a.short_rows, a.dominant_tiles) == (
-        b.partition_size, b.shared_kv, b.short_rows, b.dominant_tiles
+    assert (a.partition_size, a.shared_kv, a.short_rows, a.dominant_tiles, a.wider_partition) == (
+        b.partition_size, b.shared_kv, b.short_rows, b.dominant_tiles, b.wider_partition
     )
 
 
@@ -176,7 +176,8 @@ def test_small_buffers_grow_and_bad_arguments_are_refused() -> None:
 )  # fmt: skip
 def test_partition_of_calls_of_tiles_alone(chunks, heads, dim, want) -> None:
     """With float32 and bfloat16 pools: a size whose workspace fits the library's static scratch
-    where it is estimated an eighth faster than the general rule's; both planners alike."""
+    where it is estimated an eighth faster than the general rule's; both planners alike. A size
+    below the rule's names the rule's as the wider one, for calls with a larger maximum context."""
     contexts = np.asarray([offset + rows for rows, offset in chunks])
     positions = np.concatenate([np.arange(offset, offset + rows) for rows, offset in chunks])
     seq = np.repeat(np.arange(len(chunks)), [rows for rows, _ in chunks])
@@ -186,3 +187,5 @@ def test_partition_of_calls_of_tiles_alone(chunks, heads, dim, want) -> None:
         native = ops.plan_batch_native(seq, dim, heads, tables, contexts, 16, query_positions=positions, kv_dtype=dtype)
         _same(python, native)
         assert native.partition_size == size and native.rows.shape[0] == 0
+        rule = ops._wide_partition(contexts, heads, max(1, seq.size // contexts.size))
+        assert native.wider_partition == (rule if size < rule else 0)

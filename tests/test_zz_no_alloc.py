@@ -13,6 +13,9 @@ workspace exceeds the scratch is refused before anything is enqueued.
 
 from __future__ import annotations
 
+import dataclasses
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -29,7 +32,7 @@ def _args(batch, plan, out):
     merge = plan.merge
     flags = (_native.PKV_ATTN_SHARED_KV if plan.shared_kv else 0) | (
         _native.PKV_ATTN_SHORT_ROWS if plan.short_rows else 0
-    )
+    ) | {0: 0, 512: _native.PKV_ATTN_WIDER_512, 1024: _native.PKV_ATTN_WIDER_1024}[plan.wider_partition]
     heads, dim = batch.key_cache.shape[2], batch.key_cache.shape[3]
     return (
         out.data_ptr(), batch.queries.data_ptr(), heads * dim,
@@ -114,3 +117,64 @@ def test_a_batch_beyond_the_scratch_is_refused(device) -> None:
     need = ops.attention_workspace_bytes(4096, 8, 128, 32768, 512)
     assert need > _native.STATIC_SCRATCH_BYTES
     assert lib.pkv_paged_attention_noalloc(*args, device.index, None) == _native.PKV_ETOOBIG
+
+
+@pytest.mark.parametrize(("rows", "offset", "heads", "dim", "wider"), [(64, 1000, 8, 128, 512), (301, 1500, 12, 64, 512), (64, 2500, 99, 32, 1024)])
+def test_a_small_partition_gives_way_to_a_large_maximum_context(device, rows, offset, heads, dim, wider) -> None:
+    """The planner bounds a call of tiles alone by the contexts it sees. Under an engine's maximum
+    context the workspace of its small partitions no longer fits the scratch: the calls then run
+    the same plan at the wider size, in no more memory than that needs, with the same results."""
+    context = offset + rows
+    gen = torch.Generator(device=device).manual_seed(rows)
+    blocks = -(-context // 16)
+    normal = lambda *shape: torch.randn(shape, generator=gen, device=device)  # noqa: E731
+    table = np.zeros((1, 65536 // 16), np.int32)
+    table[0, :blocks] = np.random.default_rng(rows).permutation(blocks)
+    positions = np.arange(offset, context)
+    host = ops.plan_batch_native(np.zeros(rows, np.int64), dim, heads, table, np.asarray([context]), 16,
+                                 query_positions=positions)  # fmt: skip
+    assert host.partition_size < host.wider_partition == wider
+    maximum = next(m for m in (8192, 16384, 32768, 65536)
+                   if ops.attention_workspace_bytes(rows, heads, dim, m, host.partition_size) > _native.STATIC_SCRATCH_BYTES)  # fmt: skip
+    plan = ops.upload_batch_plan(host, device)
+    batch = SimpleNamespace(
+        queries=normal(rows, heads, dim), key_cache=normal(blocks, 16, heads, dim), value_cache=normal(blocks, 16, heads, dim),
+        query_positions=torch.from_numpy(positions.astype(np.int32)).to(device),
+        query_seq=torch.zeros(rows, dtype=torch.int32, device=device), block_tables=torch.from_numpy(table).to(device),
+        context_lens=torch.tensor([context], dtype=torch.int32, device=device), num_queries=rows, num_seqs=1,
+        scale=dim**-0.5, max_context_len=context,
+    )  # fmt: skip
+    call = lambda m, p: ops.paged_attention_ragged(  # noqa: E731
+        batch.queries, batch.query_positions, batch.query_seq, batch.key_cache, batch.value_cache, batch.block_tables,
+        batch.context_lens, batch.scale, max_context_len=m, plan=p)  # fmt: skip
+    want = call(context, plan)
+    at_wider = call(context, dataclasses.replace(plan, partition_size=wider, wider_partition=0))
+    assert float((at_wider - want).abs().max()) < 1e-5
+
+    batch.max_context_len = maximum
+    out = torch.full_like(want, float("nan"))
+    lib = _native.library()
+    stream = torch.cuda.current_stream(device).cuda_stream
+    if (need := ops.attention_workspace_bytes(rows, heads, dim, maximum, wider)) <= _native.STATIC_SCRATCH_BYTES:
+        assert lib.pkv_paged_attention_noalloc(*_args(batch, plan, out), device.index, stream) == 0
+        assert torch.equal(out, at_wider)
+    else:  # the wider size does not fit either
+        assert lib.pkv_paged_attention_noalloc(*_args(batch, plan, out), device.index, stream) == _native.PKV_ETOOBIG
+    workspace = torch.empty(need // 4, dtype=torch.float32, device=device)
+    out.fill_(float("nan"))
+    assert lib.pkv_paged_attention(*_args(batch, plan, out), workspace.data_ptr(), need, device.index, stream) == 0
+    assert torch.equal(out, at_wider)
+    del workspace
+    torch.cuda.synchronize(device)
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats(device)
+    before = torch.cuda.memory_allocated(device)
+    assert torch.equal(call(maximum, plan), at_wider)
+    assert torch.cuda.max_memory_allocated(device) - before <= need + out.numel() * 4 + (4 << 20)
+    # the flag belongs to plans of tiles alone, and names one size
+    batch.max_context_len = context
+    args = list(_args(batch, plan, out))
+    args[27] |= _native.PKV_ATTN_WIDER_512 | _native.PKV_ATTN_WIDER_1024
+    assert lib.pkv_paged_attention_noalloc(*args, device.index, stream) == _native.PKV_EINVAL
+    args[27], args[9], args[10], args[12] = _native.PKV_ATTN_WIDER_512, None, 0, -1
+    assert lib.pkv_paged_attention_noalloc(*args, device.index, stream) == _native.PKV_EINVAL
