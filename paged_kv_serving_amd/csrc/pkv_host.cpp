@@ -1474,6 +1474,19 @@ int gemm(void* handle, int64_t m, int64_t n, int64_t k, const float* a, int64_t 
 constexpr int64_t kSmallRows = 512;
 constexpr int64_t kSmallModel = 256;
 
+// Whether a small decoder's logits are its own product too. That product reads the whole embedding
+// once per 16 wanted rows, so over many rows and a large vocabulary the library's larger tiles win,
+// with the norm and the gather before them. Measured on MI355X, own product / norm + gather +
+// library, device us: d_model 128, 1,024 tiles of 16 x 64 (128 rows of 8,192) 10.3 / 11.3, 2,048
+// 18 / 14; d_model 64, 8.4 / 9.9 and 14 / 12; d_model 256, 512 tiles 9.2 / 10.5, 1,024 14.3 / 12.8,
+// 512 rows of 128,256 625 / 394. Up to two tiles of rows at any size: 16 rows of 128,256 28 / 34; a
+// whole execute_greedy() of 32 rows of 128,256 (d_model 64, 128, 256) 179 / 189, 194 / 213, 235 /
+// 275, of 64 rows 199 / 191, 224 / 216, 283 / 283.
+bool small_logits(int64_t rows, int64_t vocab, int64_t d) {
+  const int64_t tiles = ((rows + 15) / 16) * ((vocab + 63) / 64);
+  return rows <= 32 || tiles <= (d <= 128 ? 1024 : 512);
+}
+
 // Integer fields of forward()'s first argument, in order.
 enum Field {
   kDevice, kStream, kTokens, kWanted, kModel, kHeads, kHeadDim, kFf, kVocab,
@@ -1677,14 +1690,17 @@ PyObject* forward(PyObject*, PyObject* args) {
   if (failed == nullptr && W > 0) {
     float* picked = f(kPicked);
     float* logits = f(kLogits);
-    const bool ready = small ? linear(PKV_LINEAR_LOGITS, hidden, d, W, d, v[kEmbedding], d, vocab, v[kFinalNorm], logits,
-                                      vocab, nullptr, nullptr, "pkv_linear_forward (logits)")
-                             : check(g_gather_rows(picked, d, normed, d, T, ptr<const int64_t>(v[kLogitsRows]), W,
-                                                   static_cast<int32_t>(d), device, stream),
-                                     "pkv_gather_rows (logits rows)") &&
-                                   check(gemm(handle, W, vocab, d, picked, d, ptr<const float>(v[kEmbedding]), d, true,
-                                              logits, vocab),
-                                         "rocblas_sgemm (logits)");
+    const bool fused_logits = small && small_logits(W, vocab, d);
+    if (small && !fused_logits) norm(v[kFinalNorm], nullptr);
+    const bool ready =
+        fused_logits ? linear(PKV_LINEAR_LOGITS, hidden, d, W, d, v[kEmbedding], d, vocab, v[kFinalNorm], logits, vocab,
+                              nullptr, nullptr, "pkv_linear_forward (logits)")
+                     : check(g_gather_rows(picked, d, normed, d, T, ptr<const int64_t>(v[kLogitsRows]), W,
+                                           static_cast<int32_t>(d), device, stream),
+                             "pkv_gather_rows (logits rows)") &&
+                           check(gemm(handle, W, vocab, d, picked, d, ptr<const float>(v[kEmbedding]), d, true, logits,
+                                      vocab),
+                                 "rocblas_sgemm (logits)");
     if (ready && v[kGreedyOut] != 0) {
       check(g_greedy_tokens(ptr<int32_t>(v[kGreedyOut]), logits, vocab, W, vocab, device, stream), "pkv_greedy_tokens");
     }
