@@ -74,7 +74,7 @@
 //       the logits rows, their product with the tied embedding, and greedy sampling when an
 //       output address is given. The products are rocBLAS sgemm calls (the rocBLAS the process
 //       has loaded, one handle per device, used by one forward pass at a time); a small decoder's
-//       (kSmallRows, kSmallModel) are pkv_linear_forward calls, which take the norms, RoPE + append,
+//       (small_decoder) are pkv_linear_forward calls, which take the norms, RoPE + append,
 //       gate, residual adds and row lookup of the logits into the same launches. `fields` holds
 //       the integers of the Field enum below (addresses, sizes, the attention plan); `layers`
 //       one tuple of six weight addresses per layer (attn_norm, qkv, out_proj, ffn_norm,
@@ -1470,9 +1470,20 @@ int gemm(void* handle, int64_t m, int64_t n, int64_t k, const float* a, int64_t 
 // 10). Measured on MI355X, execute() with its logits back on the host, library products against
 // these: d_model 128 (4 layers, 128 rows) 280 / 205 us, 2 layers of 2 rows 146 / 87, 4 layers of
 // 512 rows 327 / 270; d_model 256 (4 layers) 80 rows 280 / 250, 288 rows 348 / 320, 432 rows 336 /
-// 309; d_model 512 16 rows 245 / 261, 288 rows 413 / 482: there the library's larger tiles win.
+// 309; d_model 512 16 rows 245 / 261, 288 rows 413 / 482: there the library's larger tiles win. They
+// also win where the products over d_ff carry the time (execute_greedy(), 4 layers): d_ff 768 at
+// d_model 256 405 / 386 (512 rows); d_ff 1,024 at d_model 128 344 / 330 (512 rows), at 256 252 / 242
+// (2 rows), 316 / 318 (256), 366 / 374 (384); d_ff 1,280 at 256 293 / 304 (128), 406 / 435 (512);
+// d_ff 1,536 at 64 266 / 266 (128) and 340 / 346 (512), at 256 430 / 469 (512).
 constexpr int64_t kSmallRows = 512;
 constexpr int64_t kSmallModel = 256;
+constexpr int64_t kSmallFf = 1024;
+constexpr int64_t kAnyRowsFf = 768;         // d_ff up to which the rows alone decide, beyond it
+constexpr int64_t kSmallRowsModel = 65536;  // rows * d_model
+bool small_decoder(int64_t rows, int64_t d, int64_t ff, int head_dim) {
+  return rows <= kSmallRows && d <= kSmallModel && d % 16 == 0 && ff % 16 == 0 && (head_dim == 32 || head_dim == 64) &&
+         (ff <= kAnyRowsFf || (ff <= kSmallFf && rows * d <= kSmallRowsModel));
+}
 
 // Whether a small decoder's logits are its own product too. That product reads the whole embedding
 // once per 16 wanted rows, so over many rows and a large vocabulary the library's larger tiles win,
@@ -1592,8 +1603,7 @@ PyObject* forward(PyObject*, PyObject* args) {
           "pkv_gather_rows (embedding)");
   }
   // A small decoder's products carry the row-wise steps around them in the same launch.
-  const bool small = g_linear != nullptr && num_layers > 0 && T <= kSmallRows && d <= kSmallModel && d % 16 == 0 &&
-                     ff % 16 == 0 && ff <= PKV_LINEAR_MAX_DEPTH && (dim == 32 || dim == 64);
+  const bool small = g_linear != nullptr && num_layers > 0 && small_decoder(T, d, ff, dim);
   if (failed == nullptr && !small) norm(num_layers > 0 ? layer[0] : v[kFinalNorm], nullptr);
   auto linear = [&](int kind, const float* input, int64_t input_stride, int64_t rows, int64_t depth, int64_t weights,
                     int64_t weight_stride, int64_t cols, int64_t norm_weight, float* output, int64_t output_stride,

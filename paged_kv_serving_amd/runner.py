@@ -15,9 +15,9 @@ enqueued by one C++ call of the host extension:
                           pass, then the split-context reduce when a context spans partitions
     rocBLAS sgemm, pkv_silu_mul : the output projection and the SwiGLU block
 
-A small decoder's products (d_model up to 256, head_dim 32 or 64, up to 512 rows) are
-``pkv_linear_forward`` launches instead, which carry the norm before them and the RoPE + append,
-gate or residual add after them.
+A small decoder's products (d_model up to 256, d_ff up to 768 or 1,024, head_dim 32 or 64, up to
+512 rows) are ``pkv_linear_forward`` launches instead, which carry the norm before them and the
+RoPE + append, gate or residual add after them.
 
 Slot mappings are computed on the host with the reference's closed form and validation
 (runner.py:149-159), so they are bit-exact with the reference by construction; they, the

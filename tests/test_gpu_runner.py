@@ -712,6 +712,25 @@ def test_attend_on_an_empty_batch_returns_no_rows(device) -> None:
     assert torch.equal(runner.key_cache, want) and runner.pending_copies == []
 
 
+def _check_one_token_rows(device, rows, **sizes) -> None:
+    """Logits and greedy tokens of ``rows`` sequences at position 0 (each attends to itself alone)
+    of a one-layer decoder against the NumPy model."""
+    config = ModelConfig(n_layers=1, max_seq_len=16, **sizes)
+    weights = random_weights(config, seed=rows)
+    runner = ModelRunner(LanguageModel(config, weights), num_blocks=rows, block_size=BLOCK_SIZE, device=device)
+    tokens = np.random.default_rng(rows).integers(0, config.vocab_size, rows)
+    batch = ExecutionBatch(tuple(BatchEntry(f"s{i}", (int(t),), (0,), (i,), 0) for i, t in enumerate(tokens)))
+    got = runner.execute(batch)
+    oracle, layer = OracleModel(config, weights), weights.layers[0]
+    hidden = oracle.embed(tokens)
+    _, _, values = oracle.project_qkv(hidden, layer, np.zeros(rows, np.int64))
+    hidden = hidden + values.reshape(rows, config.d_model) @ layer.out_proj
+    want = oracle.logits_from_hidden(hidden + oracle.feed_forward(hidden, layer))
+    assert float(np.max(np.abs(np.stack([got[f"s{i}"] for i in range(rows)]) - want))) < TOLERANCE
+    greedy = runner.execute_greedy(batch)
+    assert all(greedy[f"s{i}"] == int(np.argmax(got[f"s{i}"])) for i in range(rows))
+
+
 @pytest.mark.parametrize(
     ("d_model", "heads", "vocab", "rows"),
     [(32, 1, 2112, 496), (32, 1, 2112, 512), (256, 8, 1088, 480), (256, 8, 1088, 481), (64, 2, 40_000, 32), (64, 2, 40_000, 33)],
@@ -719,19 +738,16 @@ def test_attend_on_an_empty_batch_returns_no_rows(device) -> None:
 def test_logits_products_on_both_sides_of_their_rule(device, d_model, heads, vocab, rows) -> None:
     """A small decoder's logits come from its own fused product over up to 1,024 tiles of 16 x 64
     (512 at d_model 256) or 32 rows, else from norm, gather and library product: the last sizes of
-    one and the first of the other, against the NumPy model, with greedy tokens of those logits."""
-    config = ModelConfig(vocab_size=vocab, d_model=d_model, n_layers=1, n_heads=heads, d_ff=32, max_seq_len=16)
-    weights = random_weights(config, seed=rows)
-    runner = ModelRunner(LanguageModel(config, weights), num_blocks=rows, block_size=BLOCK_SIZE, device=device)
-    tokens = np.random.default_rng(rows).integers(0, vocab, rows)
-    batch = ExecutionBatch(tuple(BatchEntry(f"s{i}", (int(t),), (0,), (i,), 0) for i, t in enumerate(tokens)))
-    got = runner.execute(batch)
-    oracle = OracleModel(config, weights)
-    hidden = oracle.embed(tokens)
-    layer = weights.layers[0]
-    _, _, values = oracle.project_qkv(hidden, layer, np.zeros(rows, np.int64))  # position 0 attends to itself
-    hidden = hidden + values.reshape(rows, d_model) @ layer.out_proj
-    want = oracle.logits_from_hidden(hidden + oracle.feed_forward(hidden, layer))
-    assert float(np.max(np.abs(np.stack([got[f"s{i}"] for i in range(rows)]) - want))) < TOLERANCE
-    greedy = runner.execute_greedy(batch)
-    assert all(greedy[f"s{i}"] == int(np.argmax(got[f"s{i}"])) for i in range(rows))
+    one and the first of the other."""
+    _check_one_token_rows(device, rows, vocab_size=vocab, d_model=d_model, n_heads=heads, d_ff=32)
+
+
+@pytest.mark.parametrize(
+    ("d_model", "heads", "d_ff", "rows"),
+    [(256, 4, 768, 512), (256, 4, 784, 256), (256, 4, 784, 257), (32, 1, 1024, 512), (32, 1, 1040, 3), (32, 1, 64, 513),
+     (288, 9, 64, 3), (128, 1, 64, 3), (64, 2, 72, 3)],
+)  # fmt: skip
+def test_layer_products_on_both_sides_of_their_rule(device, d_model, heads, d_ff, rows) -> None:
+    """The last sizes of a small decoder's fused products and the first of the library's: d_ff 768
+    and 1,024, rows x d_model 65,536 between them, 512 rows, d_model 256, head_dim 128, odd depths."""
+    _check_one_token_rows(device, rows, vocab_size=64, d_model=d_model, n_heads=heads, d_ff=d_ff)
