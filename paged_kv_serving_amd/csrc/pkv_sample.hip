@@ -8,13 +8,11 @@
 namespace pkv {
 namespace {
 
-constexpr int kArgmaxThreads = 1024;
-constexpr int kArgmaxWaves = kArgmaxThreads / kWave;
 constexpr int kArgmaxLoads = 4;  // 16-byte loads in flight per thread
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// A candidate (value, index); index -1 marks "no element seen".
+// A candidate (value, index); index -1 marks "nothing above -inf seen".
 struct Best {
   float value;
   int32_t index;
@@ -41,36 +39,48 @@ __device__ __forceinline__ Best shfl_xor_best(const Best& b, int mask) {
 // One workgroup per row. The row's 16-byte aligned body is read kArgmaxLoads vectors per thread at
 // a time (each thread scans increasing indices, so a later element only wins by being strictly
 // greater, or by being the first NaN); the up to three elements before and after it are merged.
+// A row without any element above -inf is its first element's.
 //
-// Bound: latency and one CU's read rate, as a row is one workgroup's. With 256 threads, one 4-byte
-// load in flight each (rows of an odd vocabulary start off a 16-byte boundary), 64 rows of 50257
-// took 60.5 us a call; 1024 threads with four vectors in flight take 9.6 us.
-__global__ __launch_bounds__(kArgmaxThreads) void greedy_kernel(int32_t* __restrict__ out,
-                                                                const float* __restrict__ logits,
-                                                                int64_t row_stride, int32_t vocab) {
+// Bound: short rows by the launch and the merge of the wavefronts, long ones by one CU's read rate
+// (a row is one workgroup's), many rows by HBM. Measured, rows of an odd vocabulary starting off a
+// 16-byte boundary: 64 rows of 50257 32.7 us with 256 threads and one 4-byte load in flight each,
+// 9.2 with 1024 threads and four vectors, 5.8 with the scan's checks out of the full steps; 512 rows
+// 69.5 -> 18.6 us.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void greedy_kernel(int32_t* __restrict__ out, const float* __restrict__ logits,
+                                                          int64_t row_stride, int32_t vocab) {
+  constexpr int kWaves = kThreads / kWave;
   const int64_t row = blockIdx.x;
   const float* x = logits + row * row_stride;
-  Best best{0.f, -1};
+  Best best{-INFINITY, -1};
   auto consider = [&](float v, int32_t i) {
-    if (best.index < 0 || (isnan(v) && !isnan(best.value)) || v > best.value) best = Best{v, i};
+    if (!(v <= best.value) && !isnan(best.value)) best = Best{v, i};
+  };
+  auto consider_vector = [&](const f32x4& v, int32_t i) {
+    consider(v.x, i);
+    consider(v.y, i + 1);
+    consider(v.z, i + 2);
+    consider(v.w, i + 3);
   };
   const int32_t to_line = static_cast<int32_t>((16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15) / 4;
   const int32_t head = to_line < vocab ? to_line : vocab;  // elements before the aligned body
   const f32x4* body = reinterpret_cast<const f32x4*>(x + head);
   const int32_t quads = (vocab - head) / 4;
-  for (int32_t q0 = threadIdx.x; q0 < quads; q0 += kArgmaxLoads * kArgmaxThreads) {
+  int32_t q = threadIdx.x;
+  for (; q + (kArgmaxLoads - 1) * kThreads < quads; q += kArgmaxLoads * kThreads) {
     f32x4 v[kArgmaxLoads];
 #pragma unroll
-    for (int u = 0; u < kArgmaxLoads; ++u) v[u] = body[min(q0 + u * kArgmaxThreads, quads - 1)];
+    for (int u = 0; u < kArgmaxLoads; ++u) v[u] = body[q + u * kThreads];
 #pragma unroll
-    for (int u = 0; u < kArgmaxLoads; ++u) {
-      const int32_t q = q0 + u * kArgmaxThreads;
-      if (q >= quads) break;
-      const int32_t i = head + 4 * q;
-      consider(v[u].x, i);
-      consider(v[u].y, i + 1);
-      consider(v[u].z, i + 2);
-      consider(v[u].w, i + 3);
+    for (int u = 0; u < kArgmaxLoads; ++u) consider_vector(v[u], head + 4 * (q + u * kThreads));
+  }
+  if (q < quads) {  // the thread's last vectors, fewer than kArgmaxLoads
+    f32x4 v[kArgmaxLoads - 1];
+#pragma unroll
+    for (int u = 0; u < kArgmaxLoads - 1; ++u) v[u] = body[min(q + u * kThreads, quads - 1)];
+#pragma unroll
+    for (int u = 0; u < kArgmaxLoads - 1; ++u) {
+      if (q + u * kThreads < quads) consider_vector(v[u], head + 4 * (q + u * kThreads));
     }
   }
   // The elements outside the body, one thread each: merged, as they are not in scan order.
@@ -79,7 +89,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_kernel(int32_t* __restr
   if (static_cast<int32_t>(threadIdx.x) < outside) {
     const int32_t t = static_cast<int32_t>(threadIdx.x);
     const int32_t i = t < head ? t : tail + (t - head);
-    const Best other{x[i], i};
+    const Best other{x[i], x[i] == -INFINITY ? -1 : i};
     if (beats(other, best)) best = other;
   }
   // Merge within the wavefront, then across the wavefronts through LDS.
@@ -88,8 +98,8 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_kernel(int32_t* __restr
     const Best other = shfl_xor_best(best, mask);
     if (beats(other, best)) best = other;
   }
-  __shared__ float s_value[kArgmaxWaves];
-  __shared__ int32_t s_index[kArgmaxWaves];
+  __shared__ float s_value[kWaves];
+  __shared__ int32_t s_index[kWaves];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   if (lane == 0) {
@@ -98,13 +108,13 @@ __global__ __launch_bounds__(kArgmaxThreads) void greedy_kernel(int32_t* __restr
   }
   __syncthreads();
   if (wave == 0) {
-    Best total = lane < kArgmaxWaves ? Best{s_value[lane], s_index[lane]} : Best{0.f, -1};
+    Best total = lane < kWaves ? Best{s_value[lane], s_index[lane]} : Best{-INFINITY, -1};
 #pragma unroll
-    for (int mask = kArgmaxWaves / 2; mask > 0; mask >>= 1) {
+    for (int mask = kWaves / 2; mask > 0; mask >>= 1) {
       const Best other = shfl_xor_best(total, mask);
       if (beats(other, total)) total = other;
     }
-    if (lane == 0) out[row] = total.index;
+    if (lane == 0) out[row] = max(total.index, 0);
   }
 }
 
@@ -123,7 +133,18 @@ extern "C" int pkv_greedy_tokens(int32_t* token_ids, const float* logits, int64_
   if (num_rows > 0x7fffffff) return PKV_EUNSUPPORTED;
   DeviceGuard guard(device);
   if (!guard.ok()) return PKV_EHIP;
-  hipLaunchKernelGGL(greedy_kernel, dim3(static_cast<uint32_t>(num_rows)), dim3(kArgmaxThreads), 0,
-                     static_cast<hipStream_t>(stream), token_ids, logits, row_stride, static_cast<int32_t>(vocab_size));
-  return check_launch();
+  // Few wavefronts where a row has little to scan: each one more adds to the merge and, over many
+  // rows, to the launch. Measured (us; 64 / 128 / 512 / 1024 threads): 16 rows of 512 2.98 / 3.01 /
+  // - / 3.46, of 4099 4.14 / 3.66 / 3.78 / 4.17, of 8192 5.4 / 4.26 / 3.77 / 4.32, of 50257 20.3 /
+  // 12.0 / 5.97 / 5.69; 2048 rows of 512 3.7 / 4.1 / - / 10.6, of 4099 7.1 / 6.8 / 10.8 / 17.3; 64
+  // rows of 128256 56 / 32 / 13.3 / 10.3, 256 rows 67 / 38 / 21.7 / 22.6.
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(num_rows)), dim3(threads), 0,
+                       static_cast<hipStream_t>(stream), token_ids, logits, row_stride, static_cast<int32_t>(vocab_size));
+    return check_launch();
+  };
+  if (vocab_size <= 512) return launch(greedy_kernel<64>, 64);
+  if (vocab_size <= 4096) return launch(greedy_kernel<128>, 128);
+  if (vocab_size <= 32768 || num_rows > 128) return launch(greedy_kernel<512>, 512);
+  return launch(greedy_kernel<1024>, 1024);
 }

@@ -77,3 +77,28 @@ def test_every_alignment_and_edge_of_a_row(device, vocab) -> None:
         flat.copy_(torch.from_numpy(rows))
         got = ops.greedy_tokens(flat).cpu().numpy()
         assert np.array_equal(got, _argmax_rows(rows)), (offset, got)
+
+
+@pytest.mark.parametrize(
+    ("vocab", "count"), [(v, 8) for v in (1, 5, 510, 513, 4094, 4097, 32_767, 32_771)] + [(32_771, 130)]
+)
+def test_every_workgroup_size(device, vocab, count) -> None:
+    """Both sides of the vocabularies and row counts at which the workgroup's size changes: random
+    rows, rows of -inf alone or but for one element, ties, a NaN, and +inf before a NaN."""
+    rng = np.random.default_rng(vocab)
+    rows = rng.standard_normal((count, vocab)).astype(np.float32)
+    at = rng.integers(0, vocab, 8)
+    rows[1] = -np.inf
+    rows[2] = -np.inf
+    rows[2, at[2]] = -np.finfo(np.float32).max
+    rows[3] = 0.0
+    rows[3, ::2] = -0.0
+    rows[4, at[4]] = np.nan
+    rows[5, 0], rows[5, at[5]] = np.inf, np.nan
+    rows[6, -1] = np.inf
+    rows[7] = np.nan
+    for offset in (0, 1):
+        held = torch.zeros(rows.size + 4, device=device)[offset : offset + rows.size].view(rows.shape)
+        held.copy_(torch.from_numpy(rows))
+        got = ops.greedy_tokens(held).cpu().numpy()
+        assert np.array_equal(got, _argmax_rows(rows)), (offset, got[:8])
