@@ -144,10 +144,13 @@ def test_rms_norm_at_the_edges_of_its_row_layouts(device, dim) -> None:
             np.testing.assert_allclose(got.cpu().numpy(), want, rtol=2e-6, atol=1e-12)
 
 
-@pytest.mark.parametrize(("rows", "width"), [(1, 4), (3, 1020), (2, 1024), (2, 1028), (70_000, 4), (5, 1030)])
+@pytest.mark.parametrize(("rows", "width"), [(1, 4), (3, 1020), (2, 1024), (2, 1028), (70_000, 4), (5, 1030),
+                                             (40_001, 8), (4_097, 36), (1_025, 128), (1_026, 132), (129, 1020),
+                                             (129, 1024), (130, 1028), (65_600, 516)])  # fmt: skip
 def test_silu_mul_vectors_and_rows_past_the_grid(device, rows, width) -> None:
-    """Whole and partial chunks of 1,024 elements, more rows than the grid's 65,535, and a width
-    that takes the one-element kernel; relative 1e-6 of float64, as the oracle test."""
+    """Whole and partial chunks of 1,024 elements, several narrow rows to a workgroup (the last one
+    partly filled), more groups of rows than the grid's 65,535, and sizes and a width that take
+    the one-element kernel; relative 1e-6 of float64, as the oracle test."""
     rng = np.random.default_rng(width)
     gate_up = (4 * rng.standard_normal((rows, 2 * width))).astype(np.float32)
     got = ops.silu_mul(_to(device, gate_up), width).cpu().numpy()
