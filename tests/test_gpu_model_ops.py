@@ -123,10 +123,10 @@ def test_gather_rows_picks_rows_and_zeroes_ids_outside_the_table(device, width, 
         assert np.all(got[r, width:] == 5.0)  # nothing past the row's width is written
 
 
-@pytest.mark.parametrize("dim", [4, 256, 260, 1024, 1028, 4095, 4096, 4100, 16_384, 16_388])
+@pytest.mark.parametrize("dim", [4, 64, 68, 256, 260, 1024, 1028, 4095, 4096, 4100, 16_384, 16_388])
 def test_rms_norm_at_the_edges_of_its_row_layouts(device, dim) -> None:
-    """A wavefront, 256 or 1024 threads per row, and the scalar kernel (16,388 floats, rows off a
-    16-byte boundary), each with and without the residual add, against float64: the sum of squares
+    """A wavefront, 256 or 1024 threads per row, and the scalar kernel (up to 64 floats, 16,388,
+    rows off a 16-byte boundary), each with and without the residual add, against float64: the sum of squares
     of n terms in at least 64 partial sums, a quotient and a product stay within 2e-6."""
     rng = np.random.default_rng(dim)
     for rows, pad in ((1, 0), (5, 0), (3, 1), (4, 4)):
