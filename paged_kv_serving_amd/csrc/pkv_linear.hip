@@ -109,7 +109,8 @@ __global__ __launch_bounds__(kLinearThreads) void linear_kernel(const pkv_linear
     if constexpr (kNorm) {
 #pragma unroll
       for (int mask = 8; mask > 0; mask >>= 1) squares += __shfl_xor(squares, mask);
-      const float scale = sqrtf(squares / static_cast<float>(a.depth) + a.eps);
+      // A row of zeros stays one, also with eps 0.
+      const float scale = source >= 0 ? sqrtf(squares / static_cast<float>(a.depth) + a.eps) : 1.f;
       for (int k = 4 * t; k < a.depth; k += 64) {
         f32x4 x = *reinterpret_cast<const f32x4*>(s + k);
         const f32x4 g = *reinterpret_cast<const f32x4*>(a.norm_weight + k);

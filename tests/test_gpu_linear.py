@@ -89,6 +89,10 @@ def test_add_swiglu_and_logits(device, rows, depth, cols) -> None:
                  row_index=torch.from_numpy(wanted).to(device)) == 0  # fmt: skip
     got, n = out.cpu().numpy(), _normed(x, g)
     assert np.all(got[3] == 0)
+    assert _call(device, kind=LOGITS, input=dx, input_stride=depth, rows=18, depth=depth, cols=cols, weights=dw,
+                 weight_stride=depth, output=out, output_stride=cols, norm_weight=dg, eps=0.0, input_rows=rows,
+                 row_index=torch.from_numpy(wanted).to(device)) == 0  # fmt: skip
+    assert np.all(out.cpu().numpy()[3] == 0)  # also without an eps: no 0 / 0
     keep = np.arange(18) != 3
     want = n[wanted[keep]] @ w.T
     assert np.all(np.abs(got[keep] - want) <= _bound(n[wanted[keep]], w.T))
