@@ -579,11 +579,10 @@ def test_whole_tiles_match_the_oracle(device, dim, kv, block) -> None:
 @pytest.mark.parametrize("block", [1, 5, 16])
 @pytest.mark.parametrize("whole", [False, True], ids=["partitions", "whole"])
 def test_tiles_beside_rows_equal_tiles_alone(device, dim, block, whole) -> None:
-    """Beside row-pass rows the float32 tile pass is a persistent grid that loads key and value
-    tiles straight into LDS (or, with the dominant-tiles hint, three register-staged workgroups
-    per CU); on its own it runs one workgroup per item through registers. All form the same sums
-    in the same order, so the tile rows come out bit-identical; and they match the oracle. At
-    block_size 1 whole tiles move their staged table window."""
+    """Tiles beside row-pass rows (a call this small runs one workgroup per item, with or without
+    the dominant-tiles hint) and alone form the same sums in the same order, so the tile rows come
+    out bit-identical; and they match the oracle. At block_size 1 whole tiles move their staged
+    table window."""
     say("tile paths", dim, block, whole)
     rng = np.random.default_rng(dim * 7 + block + whole)
     max_ctx = 1400 if block == 1 else 800
@@ -639,7 +638,7 @@ def test_tiles_beside_rows_equal_tiles_alone(device, dim, block, whole) -> None:
 def test_caller_rows_reach_the_rows_the_plan_orders(device, dim, block, whole) -> None:
     """caller_rows[t] is the row of queries and out that planner row t reads and writes. With
     the queries permuted and the permutation passed, the row pass, the tile pass (alone, and at
-    block 16 beside a row pass large enough for the second stream and the direct-to-LDS grid)
+    block 16 beside a row pass large enough for the second stream and the persistent grid)
     and the reduce write bit for bit what the unpermuted call writes, into the permuted rows. A
     caller row outside the batch skips its query: its output row keeps what it held."""
     say("caller rows", dim, block, whole)
@@ -877,8 +876,7 @@ def _attention_skipping_bad_blocks(q, positions, seq_of, kc, vc, tables, context
 @pytest.mark.parametrize("bad", [-1, 10**6], ids=["negative", "past-pool"])
 def test_blocks_outside_the_pool_are_skipped_by_every_pass(device, block, bad) -> None:
     """A table entry outside [0, num_blocks) inside a visible context is never read: the row
-    pass, the tile pass beside it (direct-to-LDS stages) and the tile pass alone (registers)
-    all leave its keys out of the softmax."""
+    pass, the tile pass beside it and the tile pass alone all leave its keys out of the softmax."""
     say("bad blocks", block, bad)
     rng = np.random.default_rng(block + (bad > 0))
     dim, heads = 128, 2
@@ -1181,11 +1179,12 @@ def test_empty_inputs_leave_the_pools_alone(device) -> None:
 @pytest.mark.parametrize("dim", [32, 64, 128, 256])
 @pytest.mark.parametrize("block", [3, 16])
 def test_tiles_with_infinite_values_fall_back_to_float32_products(device, kv, dim, block) -> None:
-    """A tile's products run on exact bfloat16 pieces, which an infinity does not survive, so a
+    """A tile's products run on bfloat16 pieces, which an infinity does not survive, so a
     tile that meets one is computed with float32 products: a key of -inf (times a positive query
     component) takes no weight, an infinite value reaches the rows that see it and no other
     tile, and every other row stays within the tolerance of the float64 result. Chunks of 17, 64,
-    65 and 130 rows (parts of a wavefront, whole and split tiles) from offset 40."""
+    65 and 130 rows (parts of a wavefront) from offset 40, in one partition, in partitions of 32 and
+    64 keys of which only some meet an infinity, and as whole tiles."""
     say("infinite values", kv, dim, block)
     rng = np.random.default_rng(dim + block)
     heads, offset = 2, 40
@@ -1217,10 +1216,10 @@ def test_tiles_with_infinite_values_fall_back_to_float32_products(device, kv, di
             torch.tensor([context], dtype=torch.int32, device=device), dim**-0.5,
         )  # fmt: skip
         seq = np.zeros(rows, np.int64)
-        for end in (0, ops.TILE_WHOLE):
+        for end, partition in ((0, 0), (0, 32), (0, 64), (ops.TILE_WHOLE, 0)):
             _, tiles = ops.plan_rows(seq, dim)
             tiles[:, 3] = end
-            plan = ops.upload_plan(np.zeros((0, 2), np.int32), tiles, device)
+            plan = ops.upload_plan(np.zeros((0, 2), np.int32), tiles, device, partition_size=partition)
             got = ops.paged_attention_ragged(*args, max_context_len=context, plan=plan).cpu().numpy()
             # The wavefronts (16 rows) of the last tile that reach the infinite value's step of 32
             # keys (16 at head_dim 256) multiply it, by zero or not.
@@ -1230,7 +1229,113 @@ def test_tiles_with_infinite_values_fall_back_to_float32_products(device, kv, di
             assert np.isinf(got[-1, :, 1]).all()
             clean = np.ones(got.shape, bool)
             clean[first:, :, 1] = False
-            assert np.max(np.abs(np.where(clean, got, 0) - np.where(clean, want, 0))) < FP32_TOL, (rows, end)
+            assert np.max(np.abs(np.where(clean, got, 0) - np.where(clean, want, 0))) < FP32_TOL, (rows, end, partition)
+
+
+@pytest.mark.parametrize("kv", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim", [32, 64, 128, 256])
+def test_tiles_with_nan_and_infinite_operands(device, kv, dim) -> None:
+    """NaN in a key reaches exactly the rows that see it (a masked score is replaced), NaN in a value
+    its column of those rows (and of the rows of their wavefront that multiply it by zero), NaN or
+    an infinity in a query its row and head alone, in tiles of one partition, of several and whole.
+    A product just below the largest float32, whose rounded pieces overflow, stays a finite score:
+    the key takes all the weight, or none when it is negative."""
+    say("nan operands", kv, dim)
+    rng = np.random.default_rng(dim)
+    heads, block, rows, offset = 4, 16, 130, 40
+    context, pool = offset + rows, -(-(offset + rows) // block) + 3
+    table = rng.permutation(pool)[: -(-context // block)]
+    flat = table[np.arange(context) // block] * block + np.arange(context) % block
+    keys, values = (rng.standard_normal((pool * block, heads, dim)).astype(np.float32) for _ in range(2))
+    if kv == "bfloat16":
+        keys, values = bf16_round(keys), bf16_round(values)
+    # Scores of variance 1, as with scale dim ** -0.5: a weight's relative error is a few roundings of
+    # its score, s * 2^-24, which at scale ln 2 alone (s up to 50 at dim 256) would pass 1e-5.
+    q = (rng.standard_normal((rows, heads, dim)) * (dim**-0.5 / np.log(2.0))).astype(np.float32)
+    keys[flat[100], 0, dim // 2] = np.nan
+    values[flat[context - 1], 1, 1] = np.nan  # only the last row sees this key
+    q[7, 2, dim - 1] = np.nan
+    q[90, 2, 3] = np.inf
+    edge = np.uint32(0x5F7FFFFF).view(np.float32)  # the largest below 2^64
+    q[:, 3], keys[flat, 3] = 0.0, 0.0
+    q[:, 3, 0], q[::2, 3, 0] = edge, -edge
+    keys[flat[3], 3, 0] = bf16_round(np.asarray([edge * np.float32(1 - 2.0**-8)]))[0] if kv == "bfloat16" else edge
+    positions = np.arange(offset, context)
+    scale = np.full(heads, float(np.log(2.0)))  # 1 in base 2
+    with np.errstate(all="ignore"):
+        scores = np.einsum("thd,khd->htk", q.astype(np.float64), keys[flat].astype(np.float64)) * scale[:, None, None]
+        scores[:, np.arange(context)[None, :] > positions[:, None]] = -np.inf
+        p = np.exp(scores - scores.max(-1, keepdims=True))
+        seen = values[flat].astype(np.float64)
+        seen[context - 1, 1, 1] = 0.0
+        want = np.einsum("htk,khd->thd", p / p.sum(-1, keepdims=True), seen)
+    assert np.isnan(want[100 - offset :, 0]).all() and np.isnan(want[7, 2]).all() and np.isnan(want[90, 2]).all()
+    assert np.isfinite(np.delete(want[:, 2], (7, 90), 0)).all() and np.isfinite(want[:, [1, 3]]).all()
+    args = (
+        torch.from_numpy(q).to(device), torch.from_numpy(positions.astype(np.int32)).to(device),
+        torch.zeros(rows, dtype=torch.int32, device=device),
+        *(torch.from_numpy(a.reshape(pool, block, heads, dim)).to(device).to(getattr(torch, kv)) for a in (keys, values)),
+        torch.from_numpy(table.astype(np.int32)[None]).to(device),
+        torch.tensor([context], dtype=torch.int32, device=device), float(scale[0]),
+    )  # fmt: skip
+    for end, partition in ((0, 0), (0, 32), (0, 64), (ops.TILE_WHOLE, 0)):
+        _, tiles = ops.plan_rows(np.zeros(rows, np.int64), dim)
+        tiles[:, 3] = end
+        plan = ops.upload_plan(np.zeros((0, 2), np.int32), tiles, device, partition_size=partition)
+        got = ops.paged_attention_ragged(*args, max_context_len=context, plan=plan).cpu().numpy()
+        assert np.isnan(got[-1, 1, 1]), (end, partition)
+        clean = np.ones(got.shape, bool)
+        clean[128:, 1, 1] = False  # the last row's wavefront
+        assert np.array_equal(np.isnan(got[clean]), np.isnan(want[clean])), (end, partition)
+        assert np.nanmax(np.abs(got - want)[clean]) < FP32_TOL, (end, partition)
+
+
+@pytest.mark.parametrize("kv", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim", [32, 128])
+def test_persistent_workgroups_go_on_after_a_tile_with_infinities(device, kv, dim) -> None:
+    """Beside a full row pass a few workgroups walk all tile items: after an item that meets a key of
+    -inf and is computed with float32 products, the same workgroup's next items (of the other
+    sequence) reuse its LDS. Every row matches the float64 result."""
+    say("persistent tiles after infinities", kv, dim)
+    rng = np.random.default_rng(dim)
+    heads, block, chunk, offset, decode, context = 32, 16, 130, 40, 130, 300
+    ends = np.asarray([offset + chunk, offset + chunk] + [context] * decode)
+    need = -(-ends // block)
+    tables = np.split(rng.permutation(int(need.sum())).astype(np.int32), np.cumsum(need)[:-1])
+    padded = np.zeros((ends.size, int(need.max())), np.int32)
+    for i, t in enumerate(tables):
+        padded[i, : t.size] = t
+    keys, values = (rng.standard_normal((int(need.sum()) * block, heads, dim)).astype(np.float32) for _ in range(2))
+    if kv == "bfloat16":
+        keys, values = bf16_round(keys), bf16_round(values)
+    keys[tables[0][0] * block + 5, :, 0] = -np.inf  # sequence 0, position 5
+    seq = np.concatenate([np.repeat([0, 1], chunk), np.arange(2, 2 + decode)])
+    positions = np.concatenate([np.arange(offset, offset + chunk)] * 2 + [np.full(decode, context - 1)])
+    q = rng.standard_normal((seq.size, heads, dim)).astype(np.float32)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.5
+    want = np.zeros(q.shape)
+    for s in (0, 1, 2, 100):
+        at = (padded[s, np.arange(ends[s]) // block].astype(np.int64) * block) + np.arange(ends[s]) % block
+        mine = seq == s
+        scores = np.einsum("thd,khd->htk", q[mine].astype(np.float64), keys[at].astype(np.float64)) * dim**-0.5
+        scores[:, np.arange(ends[s])[None, :] > positions[mine][:, None]] = -np.inf
+        p = np.exp(scores - scores.max(-1, keepdims=True))
+        want[mine] = np.einsum("htk,khd->thd", p / p.sum(-1, keepdims=True), values[at].astype(np.float64))
+    checked = np.isin(seq, (0, 1, 2, 100))
+    rows, tiles = ops.plan_rows(seq, dim)
+    for end, partition in ((0, 64), (0, 0), (ops.TILE_WHOLE, 0)):
+        tiles[:, 3] = end
+        items = ops.expand_rows(rows, positions + 1, partition)
+        assert tiles.shape[0] == 6 and items.shape[0] * heads // 2 >= 2048  # the persistent grid's call
+        plan = ops.upload_plan(items, tiles, device, partition_size=partition)
+        got = ops.paged_attention_ragged(
+            torch.from_numpy(q).to(device), torch.from_numpy(positions.astype(np.int32)).to(device),
+            torch.from_numpy(seq.astype(np.int32)).to(device),
+            *(torch.from_numpy(a.reshape(-1, block, heads, dim)).to(device).to(getattr(torch, kv)) for a in (keys, values)),
+            torch.from_numpy(padded).to(device), torch.from_numpy(ends.astype(np.int32)).to(device), dim**-0.5,
+            max_context_len=context, plan=plan,
+        ).cpu().numpy()  # fmt: skip
+        assert np.max(np.abs(got[checked] - want[checked])) < FP32_TOL, (end, partition)
 
 
 @pytest.mark.parametrize("dim", [32, 64, 128, 256])
