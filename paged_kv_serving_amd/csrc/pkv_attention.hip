@@ -92,7 +92,7 @@ namespace {
 #endif
 // The tile pass at head_dim 128: the occupancy target in waves per SIMD (its VGPR budget), for
 // bfloat16 pools and the float32 products. Measured on 8 chunks of 512 rows alone, bfloat16: 3
-// waves 0.235 ms, 2 waves 0.253 ms. The split float32 tiles take 237 VGPRs, two waves: held to
+// waves 0.235 ms, 2 waves 0.253 ms. The split float32 tiles take 239 VGPRs, two waves: held to
 // 168 they spill (0.53 against 0.62 ms, before their products were interleaved).
 #ifndef PKV_TILE_REG_WAVES
 #define PKV_TILE_REG_WAVES 3
@@ -1698,8 +1698,13 @@ DeviceResources* overlap_for(int device) {
 //    as fit (60 rows 1.08 against 1.26 ms, 30 rows 0.89 against 1.23);
 //  - bfloat16: one, two or three per CU are within 2% at every balance (120 rows 0.875-0.90 ms);
 //  - float32 beside lean row workgroups (prefix sharing): the float32 products, two per CU. The
-//    split tiles' 58 KiB of LDS and 237 VGPRs leave one lean row workgroup on the CU (0.303 ms
+//    split tiles' 58 KiB of LDS and 239 VGPRs leave one lean row workgroup on the CU (0.303 ms
 //    the step against 0.271; 0.332 with one per CU, 0.292 with the passes one after the other).
+//  - float32 alone: always the split tiles. On contexts of a few dozen keys their longer start is
+//    not made up for (33 keys at head_dim 32 7.4 us against 6.7 with the float32 products, 203 keys
+//    12.4 against 11.9; 33 keys at head_dim 256 16.6 against 15.5; never at 64 and 128), but their
+//    error is smaller there too (head_dim 32, 33 keys 7e-8 against 1.3e-7, 203 keys 1.4e-7 against
+//    2.1e-7; 256, 33 keys 2.2e-7 against 2.7e-7), so short calls keep them.
 // PKV_ATTN_DOMINANT_TILES changes the grid only, never the products.
 template <typename KVT, int D>
 int launch_tiles(const Params& a, int64_t num_tiles, int64_t cus, bool lean_rows, hipStream_t stream) {

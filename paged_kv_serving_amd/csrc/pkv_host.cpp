@@ -1466,8 +1466,8 @@ int gemm(void* handle, int64_t m, int64_t n, int64_t k, const float* a, int64_t 
                       static_cast<int32_t>(lda), &zero, c, static_cast<int32_t>(ldc));
 }
 
-// Up to these sizes forward() takes pkv_linear_forward's products (7 launches a layer instead of
-// 10). Measured on MI355X, execute() with its logits back on the host, library products against
+// Up to these sizes forward() takes pkv_linear_forward's products (6 launches a layer with both
+// attention passes instead of 10). Measured on MI355X, execute() with its logits back on the host, library products against
 // these: d_model 128 (4 layers, 128 rows) 280 / 205 us, 2 layers of 2 rows 146 / 87, 4 layers of
 // 512 rows 327 / 270; d_model 256 (4 layers) 80 rows 280 / 250, 288 rows 348 / 320, 432 rows 336 /
 // 309; d_model 512 16 rows 245 / 261, 288 rows 413 / 482: there the library's larger tiles win. They

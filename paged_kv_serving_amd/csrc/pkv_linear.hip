@@ -2,7 +2,7 @@
 // RMSNorm of the input rows before the product, and after it the residual add, RoPE with the
 // slot-mapped append, or the SwiGLU gate. At the sizes this serves (up to 512 rows, d_model up
 // to 256) every launch is latency: a library product takes 4.5-6.7 us, a norm 3.2, RoPE + append
-// 3.8, a gate 2.7, whatever they compute, and a layer had nine of them.
+// 3.8, a gate 2.7, whatever they compute, and a layer had eight of them beside attention's passes.
 //
 // Products are float32 (v_mfma_f32_16x16x4f32). One workgroup computes 16 rows x 64 columns, a
 // wavefront 16 of the columns, so that even 128 rows of 384 columns are 48 workgroups. The 16 input
@@ -10,7 +10,7 @@
 // once); the weights are read once per workgroup straight into registers, 128 of the depth at a
 // time, the first of them before the rows are staged. Measured, one iteration of a 4-layer decoder
 // (d_model 128, 128 rows), logits back on the host: 286 us with the library's products and the
-// separate steps, 207 us with these (7 launches a layer in place of 10).
+// separate steps, 207 us with these (6 launches a layer with both attention passes, in place of 10).
 #include <math.h>
 
 #include "pkv_common.h"

@@ -66,8 +66,9 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
 // read and written once. Needs 16-byte aligned rows and dim <= 16 * kCache * kRowThreads / 4 floats.
 //
 // Bound: HBM (hidden and delta read, hidden and out written). A wavefront per row with 4-byte
-// accesses kept too few bytes in flight and read the row twice: 1024 rows of 4096 with the
-// residual add (67 MB) took 40.3 us, 1.7 TB/s; 256 threads a row take 11.5 us, 5.8 TB/s.
+// accesses kept too few bytes in flight and read the row twice. 1024 rows of 4096 with the residual
+// add (67 MB) over buffers that rotate through 1 GB: 52.1 us, 256 threads a row 16.7 (4.0 TB/s).
+// Over one set of buffers, which the 256 MB Infinity Cache holds between passes: 38-40 and 10-11.5.
 template <int kRowThreads, int kCache>
 __global__ __launch_bounds__(kRowThreads < kNormThreads ? kNormThreads : kRowThreads) void rms_norm_vec_kernel(
     float* out, int64_t out_stride, float* hidden, int64_t hidden_stride, const float* __restrict__ delta,
@@ -134,8 +135,9 @@ __device__ __forceinline__ float silu_product(float g, float u) {
 // vectors, rounded up) per row or chunk of a row. Grid: (chunks of a row, groups of rows), the rows
 // beyond the grid's strided.
 //
-// Bound: HBM (gate and up read, out written). One element per thread with a 64-bit division for
-// its row took 26.7 us for 1024 rows of 11008 (135 MB, 5.1 TB/s); this takes 23.6 us (5.7 TB/s).
+// Bound: HBM (gate and up read, out written). 1024 rows of 11008 (135 MB) over buffers that rotate
+// through 1.6 GB: 35.6 us with one element per thread and a 64-bit division for its row, 26.2 with
+// this (5.2 TB/s). Over one set of buffers, which the Infinity Cache mostly holds: 27.4 and 24.5.
 // Narrow rows by the workgroups: 4096 rows of 64 took 3.93 us with a workgroup each, 2.54 with one
 // element per thread.
 __global__ __launch_bounds__(kGateThreads) void silu_mul_vec_kernel(float* __restrict__ out, int64_t out_stride,

@@ -350,7 +350,8 @@ class AttentionPlan:
     exactly once. ``merge``: int32 ``[M]``, the rows whose partition results the reduce pass
     merges (None: every row, which is only correct without whole tiles). ``partition_size``
     (0: library default), ``shared_kv``, ``short_rows`` (the lighter row-pass workgroup for
-    short items) and ``dominant_tiles`` (three tile-pass workgroups per CU beside the rows)
+    short items) and ``dominant_tiles`` (up to three tile-pass workgroups per CU beside the
+    rows)
     choose the launch. ``wider_partition`` (512, 1024 or 0; plans of tiles alone): the size a call
     takes instead where the workspace at ``partition_size`` and its ``max_context_len`` would not
     fit the library's static scratch.
